@@ -1,4 +1,4 @@
-// Gated DeltaNet chunked prefill on gfx950 (WY/UT form, chunk C = 64).
+// Gated DeltaNet chunked prefill on gfx950 (UT form, chunk C = 64).
 //
 // Reference: Qwen35HybridTextBackend::run_linear_delta_prefill_gpu_batched
 // (src/models/Qwen35HybridTextBackend.cpp:1306-1508) applies the decode
@@ -7,181 +7,238 @@
 //
 // For a chunk with state S0 [dk, dv] (rows = key dims), normalisers
 // ik_t = 1/sqrt(|k_t|^2+eps), iq_t likewise, beta_t, cumulative log-decay
-// G_t = sum_{s<=t} g_t, and the raw bf16 inputs K, Q, V (exact in bf16):
+// G_t = sum_{s<=t} g_t, and the inputs K, Q, V:
 //   A[t,s]  = beta_t e^(G_t-G_s) ik_t ik_s (K K^T)[t,s]          (s < t)
 //   T       = (I + A)^-1,  To = T - I                            (fp32)
-//   W       = bf16(To diag(sw)) K + diag(sw) K,   sw = beta e^G ik
-//   U       = bf16(To diag(beta)) V + diag(beta) V
-//   D       = U - W S0
+//   R       = diag(beta) V - diag(sw) (K S0),   sw = beta e^G ik
+//   D       = R + To R
 //   O       = scale * ( fq (Q S0) + P D ),   fq = e^G iq,
 //             P[t,s] = e^(G_t-G_s) iq_t ik_s (Q K^T)[t,s]          (s <= t)
 //   S1      = e^(G_last) S0 + K^T (fk D),      fk = e^(G_last-G) ik
 // All decays are formed as exp of differences with s <= t (never a ratio),
 // so they stay in [0, 1]. T is computed in fp32 (diagonal 16x16 blocks by
-// substitution, off-diagonal blocks on the fp32 matrix cores), the diagonal
-// of T is applied in fp32, and every product that feeds the state carries
-// its inexact operands as a hi + lo pair of bf16 (x = bf16(x) + bf16(x -
-// bf16(x)), 2^-16 relative): To diag(beta) and To diag(sw) in U and W, W and
-// S in D = U - W S, and (fk D) in the state update, each as hi*hi + hi*lo +
-// lo*hi. With decays near 1 the chunk's W S nearly cancels U, and single
-// bf16 roundings there would grow the state error past 1e-3 within a few
-// thousand tokens. The output-only products (Q S, P D) use single bf16.
+// substitution, off-diagonal blocks on the fp32 matrix cores), its unit
+// diagonal is applied in fp32, and every product that feeds the state
+// carries its inexact operands as a hi + lo pair of bf16 (x = bf16(x) +
+// bf16(x - bf16(x)), 2^-16 relative): S (and K, when it is the fp32 conv
+// output) in K S0, To and R in To R, fk D (and K) in the state update, each
+// as hi*hi + hi*lo + lo*hi. With decays near 1 sw K S0 nearly cancels beta V;
+// forming that difference first, in fp32, keeps T's operand small. The
+// output-only products (Q S, P D) use single bf16 (S as hi + lo in the layer).
 //
-// The prep writes the records with nontemporal stores: each is read once,
-// by the scan, after the whole prep has run (layer prefill at config 4:
-// 258 -> 242 us, most of it in the scan's reads of them).
-//
-// Kernel 1 (deltanet_chunk_prep_kernel): one workgroup per (chunk, value
-//   head, sequence), fully parallel, three per CU (two with split inputs).
-//   K and Q tiles arrive by DMA, V rows wait in registers for the A space;
-//   it writes W, K^T, P, U and the row factors to the workspace, each
-//   in the register order of the scan's MFMA operands (16-byte loads there).
-// Kernel 2 (deltanet_chunk_scan_kernel): one 8-wave workgroup per (16-column
-//   slab of dv, value head, sequence); walks the chunks in order with its
-//   [dk x 16] state slab in registers (C layout of v_mfma_f32_16x16x32) of
-//   four "state" waves while four "output" waves form the outputs beside
-//   them; each wave prefetches its own operands of chunk c+2 into registers
-//   while chunk c computes, and D and S are exchanged through LDS.
+// Kernel 1 (deltanet_chunk_prep_kernel): one workgroup per (chunk, key head,
+//   sequence) forms what the recurrence needs and S does not enter: K, Q,
+//   K K^T and Q K^T once for the key head, then To and P for each of its
+//   value heads (four waves per value head).
+// Kernel 2 (deltanet_chunk_scan_kernel): one 8-wave workgroup per (slab of 16
+//   NT columns of dv, value head, sequence) walks the chunks in order with
+//   its state slab in registers of four "state" waves, while four "output"
+//   waves form the outputs beside them, bring the K tiles of later chunks to
+//   LDS by DMA and form the V rows.
+// T is applied to R inside the scan: storing W = T diag(sw) K and U = T
+// diag(beta) V per value head instead made its chunk record 73 KiB (now 25)
+// and both products part of the prep. Layer, T = 4096, 16 key and 32 value
+// heads: prep 113 -> 44 us, scan 103 -> 85 us, call 214 -> 152 us; the
+// recurrence alone 144 -> 106 us.
 //
 // Token/key "slot" order: every MFMA that contracts over an index whose
 // B operand is published from C-layout registers (the state rows, the
-// tokens of D) uses, within each 32-wide k-step, the order in which lane
+// tokens of R and D) uses, within each 32-wide k-step, the order in which lane
 // group g (= lane / 16) supplies k = {4g..4g+3, 16+4g..16+4g+3}. The
-// workspace stores W (over k), K^T and P (over tokens) in that order.
+// workspace stores To and P (over tokens) and Q (over key dims) in that order.
 #include "common.hpp"
 #include "deltanet_generic.hpp"
 
+#include <algorithm>
 #include <type_traits>
 
 namespace aila {
 namespace {
 
 constexpr int kC = 64;          // chunk length
-constexpr int kThreads = 256;
+constexpr int kD = 128;         // key and value head dim
+constexpr int kRB = kD * 2;     // bytes per K/Q row
+constexpr int kTile = kC * kRB; // bytes of a K or Q tile
+constexpr int kHeadThreads = 256;   // prep threads per value head
+// Scan threads: four state and four output waves, and with one column tile
+// (whose registers allow a third wave per SIMD) four helper waves.
+constexpr int scan_threads(int NT) { return NT == 1 ? 768 : 512; }
 constexpr int kNumXcd = 8;      // MI355X: 8 accelerator complex dies, one L2 each
-
-// Index held by slot e (0..7) of lane group g within a 32-wide k-step.
-__device__ __forceinline__ int slot_idx(int g, int e) { return (e < 4) ? 4 * g + e : 16 + 4 * g + (e - 4); }
 
 __device__ __forceinline__ bf16x8_t cat8x2(const u32x2& a, const u32x2& b) {
   const u32x4 r = {a[0], a[1], b[0], b[1]};
   return as_bf16x8(r);
 }
+// Low 16 bits' / high 16 bits' bf16 of element e of a packed vector, as fp32.
+template <class V>
+__device__ __forceinline__ float bf_at(const V& w, int e) {
+  return __uint_as_float((e & 1) ? (w[e >> 1] & 0xffff0000u) : (w[e >> 1] << 16));
+}
+// bf16 hi + lo of eight / four fp32 values.
+__device__ __forceinline__ void split8(const float* x, u32x4& hi, u32x4& lo) {
+  hi = u32x4{pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3]), pack_bf16x2(x[4], x[5]), pack_bf16x2(x[6], x[7])};
+  float r[8];
+#pragma unroll
+  for (int e = 0; e < 8; ++e) r[e] = x[e] - bf_at(hi, e);
+  lo = u32x4{pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3]), pack_bf16x2(r[4], r[5]), pack_bf16x2(r[6], r[7])};
+}
+__device__ __forceinline__ void split4(const f32x4& x, u32x2& hi, u32x2& lo) {
+  hi = u32x2{pack_bf16x2(x[0], x[1]), pack_bf16x2(x[2], x[3])};
+  lo = u32x2{pack_bf16x2(x[0] - bf_at(hi, 0), x[1] - bf_at(hi, 1)), pack_bf16x2(x[2] - bf_at(hi, 2), x[3] - bf_at(hi, 3))};
+}
 
-// 16-byte chunk swizzles of 256-byte LDS rows (see gqa_prefill: bit 0 from
-// row bit 0 suits ds_read_b128 row reads; bit 0 from row bit 3 suits the
-// transposed reads).
-__device__ __forceinline__ int swz_rows(int r) { return r & 15; }
-__device__ __forceinline__ int swz_tr(int r) { return ((r & 7) << 1) | ((r >> 3) & 1); }
+// K and Q tiles in LDS: rows of 256 bytes, 16-byte chunks swizzled by the row.
+// kSlot tiles (formed by the prep from the fused rows) hold each 32-wide k-step
+// in slot order, so that a row's MFMA operand is one 16-byte read; tiles DMA'd
+// from the input rows keep the key order (two 8-byte reads). Both swizzles give
+// 16 rows of one chunk distinct banks; the slot tiles' also the transposing
+// reads' four rows of four half chunks.
+template <bool kSlot>
+__device__ __forceinline__ int swz_rows(int r) {
+  return kSlot ? ((r & 3) << 2) | ((r ^ (r >> 2)) & 3) : r & 15;
+}
+// 16x16 tile (I, J), J <= I, of a packed lower triangle of tiles.
+__device__ __forceinline__ constexpr int tri(int I, int J) { return I * (I + 1) / 2 + J; }
 
-// Workspace records of one chunk. Every scan operand is stored in register
-// order - [tile][k-step][lane][16 bytes] - so that one wave load is one
-// contiguous KiB (a 16-row gather would cost the memory pipe 16 cache lines
-// per instruction). The parts that depend on the value head (its gates)
-// are kept per (sequence, value head, chunk):
-//   F  fq[C], fk[C], gamma (f32)
-//   W  [4 token tiles][4 k-steps][64][8 bf16]    W[16w+l%16][32ks + slots of l/16]
-//   WLo  the bf16 residual W - bf16(W), laid out as W
-//   P  [4 token tiles][2 k-steps][64][8 bf16]    P[16w+l%16][32s2 + slots of l/16]
-//   U  [DV/16 slabs][4 token tiles][64][4 f32]   C layout of U
-// and the parts that are copies of the key head's inputs once per
-// (sequence, key head, chunk), written by the key head's first value head
-// and read by all of them:
-//   Kt [8 key tiles][2 token k-steps][64][8 bf16] K[32s2 + slots of l/16][16dt+l%16]
-//   Q  [4 token tiles][4 k-steps][64][8 bf16]    Q[16w+l%16][32ks + slots of l/16]
-//   KtLo (split inputs only) the bf16 residual K - bf16(K), laid out as Kt
-// The key-head records follow all value-head records; the workspace sizes
-// them for Hv key heads (Hk <= Hv), so its size does not depend on Hk.
-template <int DK, int DV>
+// MFMA A/B operand over 32 tokens in slot order from a tile by transposing
+// reads: lane (g4, m16) gets M[tokens of g4][16*dt + m16].
+template <bool kSlot>
+__device__ __forceinline__ bf16x8_t tr_operand(const unsigned char* tile, int ks, int dt, int m16, int g4) {
+  const int p = m16 & 3;   // keys 4p .. 4p+3 of tile dt
+  const int chunk = kSlot ? 4 * (dt >> 1) + p : 2 * dt + (p >> 1), half = kSlot ? dt & 1 : p & 1;
+  const int r0 = ks * 32 + 4 * g4 + (m16 >> 2), r1 = r0 + 16;
+  const u32x2 lo = ds_read_tr4(tile + r0 * kRB + ((chunk ^ swz_rows<kSlot>(r0)) << 4) + (half << 3));
+  const u32x2 hi = ds_read_tr4(tile + r1 * kRB + ((chunk ^ swz_rows<kSlot>(r1)) << 4) + (half << 3));
+  return cat8x2(lo, hi);
+}
+// MFMA A operand over 32 key dims in slot order: row r of a tile.
+template <bool kSlot>
+__device__ __forceinline__ bf16x8_t row_operand(const unsigned char* tile, int ks, int r, int g4) {
+  if constexpr (kSlot) {
+    return as_bf16x8(*reinterpret_cast<const u32x4*>(tile + r * kRB + (((4 * ks + g4) ^ swz_rows<kSlot>(r)) << 4)));
+  } else {
+    const unsigned char* row = tile + r * kRB + ((g4 & 1) << 3);
+    const int c = 4 * ks + (g4 >> 1);
+    const u32x2 a = *reinterpret_cast<const u32x2*>(row + ((c ^ swz_rows<kSlot>(r)) << 4));
+    const u32x2 b = *reinterpret_cast<const u32x2*>(row + (((c + 2) ^ swz_rows<kSlot>(r)) << 4));
+    return cat8x2(a, b);
+  }
+}
+
+// Workspace records of one chunk. Scan operands that go to registers are
+// stored in register order - [tile][k-step][lane][16 bytes] - so that one wave
+// load is one contiguous KiB (a 16-row gather would cost the memory pipe 16
+// cache lines per instruction). Per (sequence, value head, chunk):
+//   F  fq[C], fk[C], beta[C], sw[C], gamma (C copies: a vector load) (f32)
+//   T  [4 token tiles][2 token k-steps][64][8 bf16]  To[16w+l%16][32s2 + slots of l/16]
+//   TLo  the bf16 residual To - bf16(To), laid out as T
+//   P  as T
+// and once per (sequence, key head, chunk):
+//   K  the K tile as it lies in LDS (row-major, swizzled 16-byte chunks)
+//   KLo (split inputs only) its bf16 residual
+//   Q  [4 token tiles][4 k-steps][64][8 bf16]        Q[16w+l%16][32ks + slots of l/16]
+// (k-step 1 of the first two token tiles of T and P is zero: neither written
+// nor read.) The key-head records follow all value-head records.
 struct ChunkRec {
   static constexpr size_t kF = 0;
-  static constexpr size_t kW = 1024;
-  static constexpr size_t kWLo = kW + size_t(kC) * DK * 2;
-  static constexpr size_t kP = kWLo + size_t(kC) * DK * 2;
-  static constexpr size_t kU = kP + size_t(kC) * kC * 2;
-  static constexpr size_t kBytes = (kU + size_t(kC) * DV * 4 + 255) / 256 * 256;
+  static constexpr size_t kT = 5 * kC * 4;
+  static constexpr size_t kTLo = kT + size_t(kC) * kC * 2;
+  static constexpr size_t kP = kTLo + size_t(kC) * kC * 2;
+  static constexpr size_t kBytes = kP + size_t(kC) * kC * 2;
 };
-template <int DK, bool kLo = false>
+template <bool kLo>
 struct KeyRec {
-  static constexpr size_t kKt = 0;
-  static constexpr size_t kQ = kKt + size_t(DK) * kC * 2;
-  static constexpr size_t kKtLo = kQ + size_t(kC) * DK * 2;
-  static constexpr size_t kBytes = (kKtLo + (kLo ? size_t(DK) * kC * 2 : 0) + 255) / 256 * 256;
+  static constexpr size_t kK = 0;
+  static constexpr size_t kQ = kK + kTile;
+  static constexpr size_t kKLo = kQ + kTile;
+  static constexpr size_t kBytes = kKLo + (kLo ? kTile : 0);
 };
+static_assert(ChunkRec::kBytes % 256 == 0 && ChunkRec::kT % 256 == 0, "records keep 256-byte alignment");
 // Key-head record (b, hk, c) of a workspace laid out for B, Hv, nch.
-template <int DK, int DV, bool kLo>
+template <bool kLo>
 __host__ __device__ __forceinline__ size_t key_rec_offset(int b, int hk, int c, int B, int Hk, int Hv, int nch) {
-  return static_cast<size_t>(B) * Hv * nch * ChunkRec<DK, DV>::kBytes +
-         ((static_cast<size_t>(b) * Hk + hk) * nch + c) * KeyRec<DK, kLo>::kBytes;
+  return static_cast<size_t>(B) * Hv * nch * ChunkRec::kBytes +
+         ((static_cast<size_t>(b) * Hk + hk) * nch + c) * KeyRec<kLo>::kBytes;
 }
 
 // ---------------------------------------------------------------------------
-// kLo: the inputs are fp32 values carried as bf16 hi planes (q, k, v) plus
-// bf16 residual tiles (q_lo, k_lo, v_lo), formed in the prep from the conv
-// of the fused rows (ConvIn). The residuals enter exactly where
-// the rounding of an input would reach the state beyond fp32 accuracy - the
-// key norms, U (its MFMA pass and diagonal term) and the K^T operand of the
-// state update (a KtLo record) - and where it would reach the outputs of
-// rows whose q.k nearly cancels (the gated RMSNorm after the layer then
-// magnifies an output far below sqrt(eps)): P = Q K^T takes Q_hi K_hi +
-// Q_hi K_lo + Q_lo K_hi and the scan's Q S takes S as hi + lo. K K^T and W
-// use the hi planes.
-template <int DK, int DV, bool kLo>
-__global__ __launch_bounds__(kThreads, 2) void deltanet_chunk_prep_kernel(
-    const bf16* __restrict__ q, const bf16* __restrict__ k, const bf16* __restrict__ v,
-    ConvIn cv,
-    const bf16* __restrict__ a, const bf16* __restrict__ bg, int ab_stride, const bf16* __restrict__ dt_bias,
-    const float* __restrict__ A_log, unsigned char* __restrict__ ws, int T, int Hk, int Hv,
-    float eps) {
-  using R = ChunkRec<DK, DV>;
-  using RK = KeyRec<DK, kLo>;
-  static_assert(DK == 128 && DV == 128, "tiles of 64 rows x 256 bytes");
-  constexpr int RB = DK * 2;       // bytes per K/Q/V row
-  constexpr int NC = DK / 8;       // 16-byte chunks per row
-  __shared__ __attribute__((aligned(1024))) unsigned char sK[kC * RB];    // K, swz_rows
-  __shared__ __attribute__((aligned(1024))) unsigned char sQA[kC * RB];   // Q (swz_rows), then A fp32 [64][64]
-  // V (swz_tr) for the split inputs; without them V waits in registers
-  // until the A space frees up, which keeps the workgroup at 49.5 KiB of
-  // LDS (three per CU)
-  __shared__ __attribute__((aligned(1024))) unsigned char sVW[kLo ? kC * RB : 16];
-  __shared__ __attribute__((aligned(16))) float sT[kC * kC];              // To, fp32 [64][64]
-  __shared__ __attribute__((aligned(16))) float sG2[kC], sGn[kC], sBeta[kC], sIk[kC], sIq[kC], sSw[kC];
-  float* sA = reinterpret_cast<float*>(sQA);
-  unsigned char* const sV = kLo ? sVW : sQA;   // the V tile for U (transposed swizzle)
-  unsigned char* sKl = reinterpret_cast<unsigned char*>(sT);   // K residual (split inputs), steps 1-3
+// kLo: the inputs are fp32 values (conv + SiLU of the fused rows, ConvIn)
+// carried as bf16 hi + residual tiles. The residuals enter where the rounding
+// of an input would reach the state beyond fp32 accuracy - the key norms,
+// K K^T, K S and K^T (fk D) - and where it would reach the outputs of rows
+// whose q.k nearly cancels (the gated RMSNorm after the layer then magnifies
+// an output far below sqrt(eps)): Q K^T takes Q_hi K_hi + Q_hi K_lo +
+// Q_lo K_hi and the scan's Q S takes S as hi + lo.
+//
+// GP value heads are formed at a time by 4 waves each; a key head with more
+// runs in passes. Its conv, norms and two products are then formed once (one
+// workgroup per value head repeated them), and GP heads' serial inversions are
+// in flight side by side: the kernel is bound by those dependent chains (about
+// 14 us at one chunk) and, over many chunks, by its ~120 MB of traffic at
+// T = 4096, Hk = 16, Hv = 32 (44 us, 2.7 TB/s; two workgroups of 67 KiB a CU).
+template <bool kLo, int GP>
+__global__ __launch_bounds__(kHeadThreads * GP, GP == 2 ? 4 : GP == 1 ? 2 : GP) void deltanet_chunk_prep_kernel(
+    const bf16* __restrict__ q, const bf16* __restrict__ k, ConvIn cv, const bf16* __restrict__ a,
+    const bf16* __restrict__ bg, int ab_stride, const bf16* __restrict__ dt_bias, const float* __restrict__ A_log,
+    unsigned char* __restrict__ ws, int T, int Hk, int Hv, float eps) {
+  using R = ChunkRec;
+  using RK = KeyRec<kLo>;
+  constexpr int kThr = kHeadThreads * GP, NW = 4 * GP;
+  constexpr int kRaw = 20 * 1024;            // raw K K^T and Q K^T tiles
+  constexpr int kTri = 10 * 1024;            // ten 16x16 fp32 tiles
+  constexpr int kTiles = (kLo ? 4 : 2) * kTile;
+  constexpr int kSmem = kTiles > kRaw + GP * 2 * kTri ? kTiles : kRaw + GP * 2 * kTri;
+  // first the input tiles, then the raw products and each head's A and To
+  __shared__ __attribute__((aligned(1024))) unsigned char smem[kSmem];
+  __shared__ __attribute__((aligned(16))) float sG2[GP][kC], sGn[GP][kC], sBeta[GP][kC], sIk[kC], sIq[kC];
+  unsigned char* const sK = smem;
+  unsigned char* const sQ = smem + kTile;
+  unsigned char* const sKl = smem + (kLo ? 2 * kTile : 0);
+  unsigned char* const sQl = smem + (kLo ? 3 * kTile : 0);
 
-  const int c = blockIdx.x, hv = blockIdx.y, b = blockIdx.z;
+  const int c = blockIdx.x, hk = blockIdx.y, b = blockIdx.z;
   const int nch = (T + kC - 1) / kC;
-  const int hk = hv / (Hv / Hk);
+  const int G = Hv / Hk;
   const int t0 = c * kC;
   const int n = min(kC, T - t0);
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int grp = wave >> 2, w4 = wave & 3;
   const int m16 = lane & 15, g4 = lane >> 4;
-  unsigned char* rec = ws + ((static_cast<size_t>(b) * Hv + hv) * nch + c) * R::kBytes;
-  // the key head's first value head writes the key-head record
-  const bool key_writer = hv % (Hv / Hk) == 0;
-  unsigned char* krec = ws + key_rec_offset<DK, DV, kLo>(b, hk, c, static_cast<int>(gridDim.z), Hk, Hv, nch);
+  unsigned char* krec = ws + key_rec_offset<kLo>(b, hk, c, static_cast<int>(gridDim.z), Hk, Hv, nch);
 
-  // ---- 1. K, Q, V tiles (rows past T are zero) ---------------------------------
-  // Split inputs (the layer): thread (cc, r0) forms 16-byte chunk cc of rows
-  // r0 .. r0+3 of each tile: conv of the 7 raw rows r0-3 .. r0+3 (rows
-  // before token 0 from the ring), SiLU, then bf16 hi and residual. Q, K and
-  // the K residual go to their tiles now; V, its residual and a second copy
-  // of the K residual wait in registers for buffers that free up later.
-  const int cc1 = tid & 15, r01 = (tid >> 4) * 4;
-  u32x4 vh1[4], vl1[4], kl1[4];
-  auto put_rows = [&](unsigned char* tile, bool trswz, const u32x4 (&x)[4]) __attribute__((always_inline)) {
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      const int r = r01 + i;
-      *reinterpret_cast<u32x4*>(tile + r * RB + ((cc1 ^ (trswz ? swz_tr(r) : swz_rows(r))) << 4)) = x[i];
+  // gates of this chunk and one value head (one wave): beta, g, prefix sum G
+  auto gates = [&](int pass) __attribute__((always_inline)) {
+    if (w4 != 0) return;
+    const int hv = hk * G + min(pass * GP + grp, G - 1);
+    float beta = 0.f, g = 0.f;
+    if (lane < n) {
+      const size_t gi = (static_cast<size_t>(b) * T + t0 + lane) * ab_stride + hv;
+      beta = 1.0f / (1.0f + expf(-bf2f(bg[gi])));
+      const float dtb = dt_bias ? bf2f(dt_bias[hv]) : 0.0f;
+      const float negA = A_log ? -expf(A_log[hv]) : -1.0f;
+      g = softplus_f(bf2f(a[gi]) + dtb) * negA;
     }
+    float Gs = g;
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      const float o = __shfl_up(Gs, off);
+      if (lane >= off) Gs += o;
+    }
+    sGn[grp][lane] = Gs;
+    sG2[grp][lane] = Gs * kLog2e;
+    sBeta[grp][lane] = beta;
   };
+
+  // ---- 1. K and Q tiles (rows past T are zero) ---------------------------------
   if constexpr (kLo) {
+    // Item (tensor, cc, r0) forms 16-byte chunk cc of rows r0 .. r0+3 of the K
+    // (tensor 0) or Q tile: conv of the 7 raw rows r0-3 .. r0+3 (rows before
+    // token 0 from the ring), SiLU, then bf16 hi and residual.
     const int head = ((cv.head % 3) + 3) % 3;
     const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
         const_cast<bf16*>(cv.qkv + static_cast<size_t>(b) * T * cv.stride), 0, T * cv.stride * 2, kBufferRsrcWord3);
+    const int cc1 = tid & 15, r01 = ((tid & 255) >> 4) * 4;
     // raw rows r0-3 .. r0+3 of 8 channels from ch0 (token rows by buffer
     // load: rows past T read as zeros; rows before token 0 from the ring)
     struct Raw { u32x4 x[7]; f32x4 rg[3][2]; };
@@ -202,18 +259,15 @@ __global__ __launch_bounds__(kThreads, 2) void deltanet_chunk_prep_kernel(
         }
       }
     };
-    // conv (4 taps) + SiLU of those rows -> bf16 hi and residual of rows r0 .. r0+3
-    auto conv_tile = [&](int c0, const Raw& in, u32x4 (&hi)[4], u32x4 (&lo)[4]) __attribute__((always_inline)) {
+    // conv (4 taps) + SiLU of those rows -> bf16 hi and residual tiles
+    auto conv_rows = [&](int c0, const Raw& in, unsigned char* th, unsigned char* tl) __attribute__((always_inline)) {
       const int ch0 = c0 + cc1 * 8;
       float w[8][4];
 #pragma unroll
       for (int v4i = 0; v4i < 4; ++v4i) {      // 16 bytes = the taps of two channels
         const u32x4 r = *reinterpret_cast<const u32x4*>(cv.w + static_cast<size_t>(ch0) * 4 + v4i * 8);
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const uint32_t word = r[e >> 1];
-          w[2 * v4i + (e >> 2)][e & 3] = __uint_as_float((e & 1) ? (word & 0xffff0000u) : (word << 16));
-        }
+        for (int e = 0; e < 8; ++e) w[2 * v4i + (e >> 2)][e & 3] = bf_at(r, e);
       }
       float x[7][8];
 #pragma unroll
@@ -241,759 +295,765 @@ __global__ __launch_bounds__(kThreads, 2) void deltanet_chunk_prep_kernel(
           const float sg = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-acc * kLog2e));
           y[e] = (r01 + i < n) ? acc * sg : 0.f;
         }
-        const u32x4 h = {pack_bf16x2(y[0], y[1]), pack_bf16x2(y[2], y[3]), pack_bf16x2(y[4], y[5]),
-                         pack_bf16x2(y[6], y[7])};
-        float rsd[8];
-#pragma unroll
-        for (int e = 0; e < 8; ++e)
-          rsd[e] = y[e] - __uint_as_float((e & 1) ? (h[e >> 1] & 0xffff0000u) : (h[e >> 1] << 16));
-        hi[i] = h;
-        lo[i] = u32x4{pack_bf16x2(rsd[0], rsd[1]), pack_bf16x2(rsd[2], rsd[3]), pack_bf16x2(rsd[4], rsd[5]),
-                      pack_bf16x2(rsd[6], rsd[7])};
+        u32x4 h, l;
+        split8(y, h, l);
+        // keys 8 cc1 .. + 3 and + 4 .. 7 go to slots of lane groups g and g + 1
+        const int r = r01 + i, g = 4 * (cc1 >> 2) + 2 * (cc1 & 1), half = ((cc1 >> 1) & 1) << 3;
+        const int a0 = r * kRB + ((g ^ swz_rows<kLo>(r)) << 4) + half, a1 = r * kRB + (((g + 1) ^ swz_rows<kLo>(r)) << 4) + half;
+        *reinterpret_cast<u32x2*>(th + a0) = u32x2{h[0], h[1]};
+        *reinterpret_cast<u32x2*>(th + a1) = u32x2{h[2], h[3]};
+        *reinterpret_cast<u32x2*>(tl + a0) = u32x2{l[0], l[1]};
+        *reinterpret_cast<u32x2*>(tl + a1) = u32x2{l[2], l[3]};
       }
     };
-    const int qd = Hk * DK;
-    // each tile's rows are in flight while the previous tile is formed
-    Raw ra, rb;
-    load_rows(hk * DK, ra);
-    load_rows(qd + hk * DK, rb);
-    u32x4 hi1[4], lo1[4];
-    conv_tile(hk * DK, ra, hi1, lo1);            // Q; its residual takes the V buffer until P is formed
-    put_rows(sQA, false, hi1);
-    put_rows(sVW, false, lo1);
-    load_rows(2 * qd + hv * DV, ra);
-    conv_tile(qd + hk * DK, rb, hi1, kl1);       // K; its residual first goes to the To buffer
-    put_rows(sK, false, hi1);
-    put_rows(sKl, false, kl1);
-    conv_tile(2 * qd + hv * DV, ra, vh1, vl1);   // V
+    const int qc0 = hk * kD, kc0 = Hk * kD + hk * kD;   // first q / k channel
+    if constexpr (GP == 1) {
+      Raw ra, rb;
+      load_rows(kc0, ra);
+      load_rows(qc0, rb);
+      gates(0);
+      conv_rows(kc0, ra, sK, sKl);
+      conv_rows(qc0, rb, sQ, sQl);
+    } else {
+      Raw ra;
+      if (wave < 8) load_rows(wave < 4 ? kc0 : qc0, ra);
+      gates(0);
+      if (wave < 4) conv_rows(kc0, ra, sK, sKl);
+      else if (wave < 8) conv_rows(qc0, ra, sQ, sQl);
+    }
   } else {
-    const int kq_row = Hk * DK * 2, v_row = Hv * DV * 2;   // source row strides (bytes)
-    const u32x4 rk = buffer_rsrc(k + (static_cast<size_t>(b) * T + t0) * Hk * DK + hk * DK, (n - 1) * kq_row + RB);
-    const u32x4 rq = buffer_rsrc(q + (static_cast<size_t>(b) * T + t0) * Hk * DK + hk * DK, (n - 1) * kq_row + RB);
-    const __amdgpu_buffer_rsrc_t rv = __builtin_amdgcn_make_buffer_rsrc(
-        const_cast<bf16*>(v + (static_cast<size_t>(b) * T + t0) * Hv * DV + hv * DV), 0, (n - 1) * v_row + RB,
-        kBufferRsrcWord3);
-#pragma unroll
-    for (int i = 0; i < kC * NC / kThreads; ++i) {
-      const int slot = i * 4 + wave;                       // wave-contiguous KiB
+    const int row = Hk * kRB;   // source row stride (bytes)
+    const size_t off = (static_cast<size_t>(b) * T + t0) * Hk * kD + hk * kD;
+    const u32x4 rk = buffer_rsrc(k + off, (n - 1) * row + kRB);
+    const u32x4 rq = buffer_rsrc(q + off, (n - 1) * row + kRB);
+    for (int slot = wave; slot < kTile / 1024; slot += NW) {      // wave-contiguous KiB
       const int p = slot * 64 + lane;
-      const int r = p / NC, cc = p % NC;
-      dma16_to_lds(rk, r * kq_row + ((cc ^ swz_rows(r)) << 4), sK + slot * 1024);
-      dma16_to_lds(rq, r * kq_row + ((cc ^ swz_rows(r)) << 4), sQA + slot * 1024);
+      const int r = p / (kD / 8), cc = p % (kD / 8);
+      dma16_to_lds(rk, r * row + ((cc ^ swz_rows<kLo>(r)) << 4), sK + slot * 1024);
+      dma16_to_lds(rq, r * row + ((cc ^ swz_rows<kLo>(r)) << 4), sQ + slot * 1024);
     }
-    // V rows r01 .. r01+3, chunk cc1, into registers (rows past T read as zeros)
-#pragma unroll
-    for (int i = 0; i < 4; ++i)
-      vh1[i] = __builtin_bit_cast(u32x4, __builtin_amdgcn_raw_buffer_load_b128(rv, (r01 + i) * v_row + cc1 * 16, 0, 0));
-  }
-  // gates of this chunk (wave 0, overlapping the DMA): beta, g, prefix sum G
-  if (wave == 0) {
-    float beta = 0.f, g = 0.f;
-    if (lane < n) {
-      const size_t gi = (static_cast<size_t>(b) * T + t0 + lane) * ab_stride + hv;
-      beta = 1.0f / (1.0f + expf(-bf2f(bg[gi])));
-      const float dtb = dt_bias ? bf2f(dt_bias[hv]) : 0.0f;
-      const float negA = A_log ? -expf(A_log[hv]) : -1.0f;
-      g = softplus_f(bf2f(a[gi]) + dtb) * negA;
-    }
-    float G = g;
-#pragma unroll
-    for (int off = 1; off < 64; off <<= 1) {
-      const float o = __shfl_up(G, off);
-      if (lane >= off) G += o;
-    }
-    sGn[lane] = G;
-    sG2[lane] = G * kLog2e;
-    sBeta[lane] = beta;
+    gates(0);
   }
   __builtin_amdgcn_s_waitcnt(vmcnt_imm<0>());
   __syncthreads();
 
   auto row_chunk = [&](const unsigned char* tile, int r, int cs) __attribute__((always_inline)) {
-    return *reinterpret_cast<const u32x4*>(tile + r * RB + ((cs ^ swz_rows(r)) << 4));
+    return *reinterpret_cast<const u32x4*>(tile + r * kRB + ((cs ^ swz_rows<kLo>(r)) << 4));
   };
-  // ---- 2. row norms: 4 threads per row ------------------------------------------
-  {
-    const int r = tid >> 2, part = tid & 3;
-    float sk = 0.f, sq = 0.f;
-    if constexpr (kLo) {
-      // |k|^2 and |q|^2 of the fp32 key and query, hi + lo
-      float hi[8], lo[8];
+  // ---- 2. raw products: jobs 0..9 (K K^T), 10..19 (Q K^T), tile (ti, tj), both
+  //      transposed (rows s of tile tj, columns t of tile ti), so that a lane
+  //      holds four consecutive s of one t.
+  constexpr int kJobs = 20, JP = (kJobs + NW - 1) / NW;
+  f32x4 prod[JP];
 #pragma unroll
-      for (int cc = 0; cc < NC / 4; ++cc) {
-        unpack8(row_chunk(sK, r, part * (NC / 4) + cc), hi);
-        unpack8(row_chunk(sKl, r, part * (NC / 4) + cc), lo);
+  for (int i = 0; i < JP; ++i) {
+    const int job = wave + NW * i;
+    prod[i] = f32x4{0.f, 0.f, 0.f, 0.f};
+    if (job < kJobs) {
+      int tj = job < 10 ? job : job - 10, ti = 0;
+      while (tj > ti) { tj -= ti + 1; ++ti; }
+      const unsigned char* X = job < 10 ? sK : sQ;
+      const unsigned char* Xl = job < 10 ? sKl : sQl;
 #pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float x = r < n ? hi[e] + lo[e] : 0.f;
-          sk = fmaf(x, x, sk);
-        }
-        unpack8(row_chunk(sQA, r, part * (NC / 4) + cc), hi);
-        unpack8(row_chunk(sVW, r, part * (NC / 4) + cc), lo);
-#pragma unroll
-        for (int e = 0; e < 8; ++e) {
-          const float x = hi[e] + lo[e];
-          sq = fmaf(x, x, sq);
-        }
-      }
-    }
-#pragma unroll
-    for (int cc = 0; cc < NC / 4; ++cc) {
-      float kf[8], qf[8];
-      unpack8(row_chunk(sK, r, part * (NC / 4) + cc), kf);
-      unpack8(row_chunk(sQA, r, part * (NC / 4) + cc), qf);
-#pragma unroll
-      for (int e = 0; e < 8; ++e) {
-        if constexpr (!kLo) {
-          sk = fmaf(kf[e], kf[e], sk);
-          sq = fmaf(qf[e], qf[e], sq);
-        }
-      }
-    }
-    sk += __shfl_xor(sk, 1);
-    sk += __shfl_xor(sk, 2);
-    sq += __shfl_xor(sq, 1);
-    sq += __shfl_xor(sq, 2);
-    if (part == 0) {
-      const float ik = 1.0f / sqrtf(sk + eps);
-      sIk[r] = ik;
-      sIq[r] = 1.0f / sqrtf(sq + eps);
-      sSw[r] = sBeta[r] * expf(sGn[r]) * ik;
-    }
-  }
-  __syncthreads();
-
-  // ---- 2b. Q in register order for the scan (before its tile becomes A) ------
-  if (key_writer) {
-    u32x4* Qout = reinterpret_cast<u32x4*>(krec + RK::kQ);
-#pragma unroll
-    for (int i = 0; i < kC * DK * 2 / 16 / kThreads; ++i) {
-      const int o = i * kThreads + tid;             // [tile][k-step][lane]
-      const int l = o & 63, ks = (o >> 6) & 3, tw = o >> 8;
-      const int r = tw * 16 + (l & 15), g = l >> 4;
-      const int k0 = ks * 32 + 4 * g, k1 = k0 + 16;   // slots 0..3 and 4..7
-      const int a0 = r * RB + (((k0 >> 3) ^ swz_rows(r)) << 4) + ((k0 & 7) << 1);
-      const int a1 = r * RB + (((k1 >> 3) ^ swz_rows(r)) << 4) + ((k1 & 7) << 1);
-      const u32x2 lo = *reinterpret_cast<const u32x2*>(sQA + a0);
-      const u32x2 hi = *reinterpret_cast<const u32x2*>(sQA + a1);
-      __builtin_nontemporal_store(u32x4{lo[0], lo[1], hi[0], hi[1]}, &Qout[o]);
-    }
-  }
-
-  // ---- 3. A = masked K K^T (LDS, fp32) and P (register order, global) -------
-  // Jobs 0..9: K K^T tiles (ti >= tj). Jobs 10..17: P of token tile ti over
-  // s k-step s2, formed as P^T (operands swapped) for the two s tiles 2*s2,
-  // 2*s2+1, so that each lane holds the 8 values of its register-order slot.
-  // Wave w takes jobs w, w+4, ...; all products first (Q is read), then the
-  // epilogues.
-  f32x4 acc3[5][2];
-#pragma unroll
-  for (int i = 0; i < 5; ++i) {
-    const int job = wave + 4 * i;
-    acc3[i][0] = acc3[i][1] = f32x4{0.f, 0.f, 0.f, 0.f};
-    if (job < 10) {
-      int tl = job, ti = 0;
-      while (tl > ti) { tl -= ti + 1; ++ti; }
-      const int tj = tl;
-#pragma unroll
-      for (int ks = 0; ks < DK / 32; ++ks) {
-        const bf16x8_t ki = as_bf16x8(row_chunk(sK, ti * 16 + m16, ks * 4 + g4));
-        const bf16x8_t kj = as_bf16x8(row_chunk(sK, tj * 16 + m16, ks * 4 + g4));
-        acc3[i][0] = mfma16x16x32(ki, kj, acc3[i][0]);
+      for (int ks = 0; ks < kD / 32; ++ks) {
+        const bf16x8_t ka = as_bf16x8(row_chunk(sK, tj * 16 + m16, ks * 4 + g4));
+        const bf16x8_t xb = as_bf16x8(row_chunk(X, ti * 16 + m16, ks * 4 + g4));
+        prod[i] = mfma16x16x32(ka, xb, prod[i]);
         if constexpr (kLo) {
-          acc3[i][0] = mfma16x16x32(ki, as_bf16x8(row_chunk(sKl, tj * 16 + m16, ks * 4 + g4)), acc3[i][0]);
-          acc3[i][0] = mfma16x16x32(as_bf16x8(row_chunk(sKl, ti * 16 + m16, ks * 4 + g4)), kj, acc3[i][0]);
-        }
-      }
-    } else if (job < 18) {
-      const int ti = (job - 10) >> 1, s2 = (job - 10) & 1;
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int tj = 2 * s2 + h;
-        if (tj <= ti) {
-#pragma unroll
-          for (int ks = 0; ks < DK / 32; ++ks) {
-            const bf16x8_t kb = as_bf16x8(row_chunk(sK, tj * 16 + m16, ks * 4 + g4));
-            const bf16x8_t qb = as_bf16x8(row_chunk(sQA, ti * 16 + m16, ks * 4 + g4));
-            acc3[i][h] = mfma16x16x32(kb, qb, acc3[i][h]);
-            if constexpr (kLo) {
-              // split inputs: the rounding of q and k would otherwise reach
-              // the outputs of rows whose q.k nearly cancels
-              acc3[i][h] = mfma16x16x32(as_bf16x8(row_chunk(sKl, tj * 16 + m16, ks * 4 + g4)), qb, acc3[i][h]);
-              acc3[i][h] = mfma16x16x32(kb, as_bf16x8(row_chunk(sVW, ti * 16 + m16, ks * 4 + g4)), acc3[i][h]);
-            }
-          }
+          prod[i] = mfma16x16x32(as_bf16x8(row_chunk(sKl, tj * 16 + m16, ks * 4 + g4)), xb, prod[i]);
+          prod[i] = mfma16x16x32(ka, as_bf16x8(row_chunk(Xl, ti * 16 + m16, ks * 4 + g4)), prod[i]);
         }
       }
     }
   }
-  __syncthreads();   // Q is no longer read: its space becomes A
-  if constexpr (kLo) put_rows(sVW, true, vh1);   // the query residual is spent: V into its buffer
-  auto v4 = [&](const float* arr, int i0) __attribute__((always_inline)) { return *reinterpret_cast<const f32x4*>(arr + i0); };
-  u32x4* Pout = reinterpret_cast<u32x4*>(rec + R::kP);
+  // ---- 3. row norms: 4 threads per row of the K and the Q tile -------------------
+  for (int it = tid; it < 2 * 4 * kC; it += kThr) {
+    const int r = (it & 255) >> 2, part = it & 3;
+    const unsigned char* X = it < 256 ? sK : sQ;
+    const unsigned char* Xl = it < 256 ? sKl : sQl;
+    float ss = 0.f;
 #pragma unroll
-  for (int i = 0; i < 5; ++i) {
-    const int job = wave + 4 * i;
-    if (job < 10) {
-      int tl = job, ti = 0;
-      while (tl > ti) { tl -= ti + 1; ++ti; }
-      const int tj = tl;
-      const int s = tj * 16 + m16, t0r = ti * 16 + g4 * 4;
-      const f32x4 bt = v4(sBeta, t0r), ikt = v4(sIk, t0r), g2t = v4(sG2, t0r);
-      const float iks = sIk[s], g2s = sG2[s];
+    for (int cc = 0; cc < kD / 32; ++cc) {
+      float x[8];
+      unpack8(row_chunk(X, r, part * (kD / 32) + cc), x);
+      if constexpr (kLo) {
+        float l[8];
+        unpack8(row_chunk(Xl, r, part * (kD / 32) + cc), l);
 #pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        const int t = t0r + j;
-        sA[t * kC + s] = (s < t) ? bt[j] * ikt[j] * iks * fast_exp2(g2t[j] - g2s) * acc3[i][0][j] : 0.f;
+        for (int e = 0; e < 8; ++e) x[e] += l[e];
       }
-    } else if (job < 18) {
-      const int ti = (job - 10) >> 1, s2 = (job - 10) & 1;
-      const int t = ti * 16 + m16;
-      const float iqt = sIq[t], g2t = sG2[t];
-      float pv[8];
 #pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int s0 = s2 * 32 + h * 16 + 4 * g4;
-        const f32x4 iks = v4(sIk, s0), g2s = v4(sG2, s0);
-#pragma unroll
-        for (int j = 0; j < 4; ++j)
-          pv[4 * h + j] = (s0 + j <= t) ? iqt * iks[j] * fast_exp2(g2t - g2s[j]) * acc3[i][h][j] : 0.f;
-      }
-      __builtin_nontemporal_store(u32x4{pack_bf16x2(pv[0], pv[1]), pack_bf16x2(pv[2], pv[3]),
-                                              pack_bf16x2(pv[4], pv[5]), pack_bf16x2(pv[6], pv[7])}, &Pout[(ti * 2 + s2) * 64 + lane]);
+      for (int e = 0; e < 8; ++e) ss = fmaf(x[e], x[e], ss);
     }
+    ss += __shfl_xor(ss, 1);
+    ss += __shfl_xor(ss, 2);
+    if (part == 0) (it < 256 ? sIk : sIq)[r] = 1.0f / sqrtf(ss + eps);
   }
+  // ---- 4. key-head record: K tile image(s), Q in register order ------------------
+  for (int o = tid; o < kTile / 16; o += kThr) {
+    __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(sK + o * 16), reinterpret_cast<u32x4*>(krec + RK::kK) + o);
+    if constexpr (kLo)
+      __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(sKl + o * 16), reinterpret_cast<u32x4*>(krec + RK::kKLo) + o);
+    // [token tile][k-step][lane]
+    const int l = o & 63;
+    __builtin_nontemporal_store(__builtin_bit_cast(u32x4, row_operand<kLo>(sQ, (o >> 6) & 3, (o >> 8) * 16 + (l & 15), l >> 4)),
+                                reinterpret_cast<u32x4*>(krec + RK::kQ) + o);
+  }
+  __syncthreads();   // the tiles are read: their space becomes the raw products, A and To
+  f32x4* const raw = reinterpret_cast<f32x4*>(smem);
+#pragma unroll
+  for (int i = 0; i < JP; ++i)
+    if (wave + NW * i < kJobs) raw[(wave + NW * i) * 64 + lane] = prod[i];
   __syncthreads();
 
-  // ---- 4. To = (I + A)^-1 - I ---------------------------------------------------
-  // 4a. diagonal block w by substitution: lane (g4, m16) owns column m16 and
-  //     the partial sums over rows m = 4*g4 .. 4*g4+3 of the block.
-  {
-    const int base = wave * 16, j = m16;
-    float xl[4];
+  float* const sA = reinterpret_cast<float*>(smem + kRaw + grp * 2 * kTri);
+  float* const sT = sA + kTri / 4;
+  for (int pass = 0; pass * GP < G; ++pass) {
+    const bool live = pass * GP + grp < G;
+    const int hv = hk * G + min(pass * GP + grp, G - 1);
+    unsigned char* rec = ws + ((static_cast<size_t>(b) * Hv + hv) * nch + c) * R::kBytes;
+    // ---- 5. A (LDS, packed tiles) and P (register order) with this head's gates --
 #pragma unroll
-    for (int kk = 0; kk < 4; ++kk) xl[kk] = (4 * g4 + kk == j) ? 1.f : 0.f;
+    for (int i = 0; i < 4; ++i) {
+      const int job = w4 + 4 * i;
+      if (job < 10) {
+        int tj = job, ti = 0;
+        while (tj > ti) { tj -= ti + 1; ++ti; }
+        const int t = ti * 16 + m16, s0 = tj * 16 + 4 * g4;
+        const f32x4 x = raw[job * 64 + lane];
+        const f32x4 iks = *reinterpret_cast<const f32x4*>(sIk + s0), g2s = *reinterpret_cast<const f32x4*>(sG2[grp] + s0);
+        const float f = sBeta[grp][t] * sIk[t], g2t = sG2[grp][t];
+        f32x4 r;
 #pragma unroll
-    for (int i = 1; i < 16; ++i) {
-      const f32x4 arow = *reinterpret_cast<const f32x4*>(&sA[(base + i) * kC + base + 4 * g4]);
-      float part = arow[0] * xl[0];
+        for (int j = 0; j < 4; ++j) r[j] = (s0 + j < t) ? f * iks[j] * fast_exp2(g2t - g2s[j]) * x[j] : 0.f;
+        *reinterpret_cast<f32x4*>(sA + job * 256 + m16 * 16 + 4 * g4) = r;
+      } else if (live) {
+        // P jobs (ti, s2): (0,0) (1,0) (2,0) (2,1) (3,0) (3,1)
+        const int pj = job - 10, ti = pj < 2 ? pj : 2 + ((pj - 2) >> 1), s2 = pj < 2 ? 0 : (pj & 1);
+        const int t = ti * 16 + m16;
+        const float iqt = sIq[t], g2t = sG2[grp][t];
+        float pv[8];
 #pragma unroll
-      for (int kk = 1; kk < 4; ++kk) part = fmaf(arow[kk], xl[kk], part);   // A[i][m] = 0 for m >= i
-      const float sum = xrow4_sum(part);
-      const float xi = (i > j) ? -sum : ((i == j) ? 1.f : 0.f);
+        for (int h = 0; h < 2; ++h) {
+          const int tj = 2 * s2 + h, s0 = tj * 16 + 4 * g4;
+          const f32x4 x = raw[(10 + tri(ti, min(tj, ti))) * 64 + lane];
+          const f32x4 iks = *reinterpret_cast<const f32x4*>(sIk + s0), g2s = *reinterpret_cast<const f32x4*>(sG2[grp] + s0);
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            pv[4 * h + j] = (s0 + j <= t) ? iqt * iks[j] * fast_exp2(g2t - g2s[j]) * x[j] : 0.f;
+        }
+        __builtin_nontemporal_store(u32x4{pack_bf16x2(pv[0], pv[1]), pack_bf16x2(pv[2], pv[3]),
+                                          pack_bf16x2(pv[4], pv[5]), pack_bf16x2(pv[6], pv[7])},
+                                    reinterpret_cast<u32x4*>(rec + R::kP) + (ti * 2 + s2) * 64 + lane);
+      }
+    }
+    // row factors
+    if (live && w4 == 3) {
+      float* F = reinterpret_cast<float*>(rec + R::kF);
+      const float Gt = sGn[grp][lane], Glast = sGn[grp][n - 1], ik = sIk[lane], beta = sBeta[grp][lane];
+      F[lane] = (lane < n) ? expf(Gt) * sIq[lane] : 0.f;                   // fq
+      F[kC + lane] = (lane < n) ? expf(Glast - Gt) * ik : 0.f;             // fk
+      F[2 * kC + lane] = beta;
+      F[3 * kC + lane] = beta * expf(Gt) * ik;                             // sw
+      F[4 * kC + lane] = expf(Glast);                                      // gamma
+    }
+    __syncthreads();
+
+    // ---- 6. To = (I + A)^-1 - I -----------------------------------------------
+    // 6a. diagonal block w4 by substitution: lane (g4, m16) owns column m16 and
+    //     the partial sums over rows m = 4*g4 .. 4*g4+3 of the block.
+    {
+      const float* At = sA + tri(w4, w4) * 256;
+      const int j = m16;
+      float xl[4];
+#pragma unroll
+      for (int kk = 0; kk < 4; ++kk) xl[kk] = (4 * g4 + kk == j) ? 1.f : 0.f;
+#pragma unroll
+      for (int i = 1; i < 16; ++i) {
+        const f32x4 arow = *reinterpret_cast<const f32x4*>(At + i * 16 + 4 * g4);
+        float part = arow[0] * xl[0];
+#pragma unroll
+        for (int kk = 1; kk < 4; ++kk) part = fmaf(arow[kk], xl[kk], part);   // A[i][m] = 0 for m >= i
+        const float sum = xrow4_sum(part);
+        const float xi = (i > j) ? -sum : ((i == j) ? 1.f : 0.f);
+#pragma unroll
+        for (int kk = 0; kk < 4; ++kk)
+          if (4 * g4 + kk == i) xl[kk] = xi;
+      }
 #pragma unroll
       for (int kk = 0; kk < 4; ++kk)
-        if (4 * g4 + kk == i) xl[kk] = xi;
-    }
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) {
-      const int i = 4 * g4 + kk;
-      sT[(base + i) * kC + base + j] = (i > j) ? xl[kk] : 0.f;
-    }
-  }
-  // strictly-upper blocks of To are zero
-  for (int idx = tid; idx < kC * kC; idx += kThreads) {
-    const int r = idx / kC, cc = idx % kC;
-    if ((cc >> 4) > (r >> 4)) sT[idx] = 0.f;
-  }
-  __syncthreads();
-  // 4b. off-diagonal blocks by distance d on the fp32 matrix cores:
-  //     T_IJ = -(I + To_II) R,  R = sum_{M=J}^{I-1} A_IM T_MJ,  T_JJ = I + To_JJ.
-  // 16x16x16 products on v_mfma_f32_16x16x4f32 with the k index permuted so
-  // that at step kk lane group g supplies k = 4g + kk: the A operand of the
-  // four steps is one float4 of row m16, and a 16x16 block held in C layout
-  // (lane (g, m16) has rows 4g..4g+3 of column m16) is directly the B
-  // operand of the four steps.
-  auto prod = [&](f32x4 acc, const float* X, int xr, int xc, const f32x4& yb) __attribute__((always_inline)) {
-    const f32x4 xa = *reinterpret_cast<const f32x4*>(&X[(xr + m16) * kC + xc + 4 * g4]);
-#pragma unroll
-    for (int kk = 0; kk < 4; ++kk) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[kk], yb[kk], acc, 0, 0, 0);
-    return acc;
-  };
-  auto cblock = [&](const float* Y, int yr, int yc) __attribute__((always_inline)) {   // C layout of a block
-    f32x4 r;
-#pragma unroll
-    for (int j = 0; j < 4; ++j) r[j] = Y[(yr + 4 * g4 + j) * kC + yc + m16];
-    return r;
-  };
-  for (int d = 1; d < 4; ++d) {
-    if (wave < 4 - d) {
-      const int J = wave, I = J + d;
-      f32x4 r = cblock(sA, I * 16, J * 16);                                 // A_IJ (identity part of T_JJ)
-      r = prod(r, sA, I * 16, J * 16, cblock(sT, J * 16, J * 16));          // + A_IJ To_JJ
-      for (int M = J + 1; M < I; ++M) r = prod(r, sA, I * 16, M * 16, cblock(sT, M * 16, J * 16));
-      const f32x4 tr = prod(r, sT, I * 16, I * 16, r);                      // R + To_II R
-#pragma unroll
-      for (int jj = 0; jj < 4; ++jj) sT[(I * 16 + 4 * g4 + jj) * kC + J * 16 + m16] = -tr[jj];
+        sT[tri(w4, w4) * 256 + (4 * g4 + kk) * 16 + j] = (4 * g4 + kk > j) ? xl[kk] : 0.f;
     }
     __syncthreads();
-  }
-  // The A space is free once To is formed: the V residual (split inputs)
-  // or V itself goes there
-  if constexpr (kLo) put_rows(sQA, true, vl1);
-  else put_rows(sQA, true, vh1);
-  __syncthreads();
-
-  // ---- 5. U = bf16(To diag(beta)) V + diag(beta) V, then W likewise with K ----
-  // wave w owns token tile w; A operands in slot order over s, B operands by
-  // transposing reads of the V / K tiles in the same order.
-  const int ti = wave;
-  const int nks = ti / 2 + 1;                     // k-steps of 32 tokens up to the diagonal
-  // (To diag(fac)) in slot order as a hi + lo pair of bf16 operands
-  auto a_operand = [&](int ks, const float* fac, bf16x8_t& hi, bf16x8_t& lo) __attribute__((always_inline)) {
-    const int t = ti * 16 + m16;
-    float f[8], r[8];
+    // 6b. off-diagonal blocks by distance d on the fp32 matrix cores:
+    //     T_IJ = -(I + To_II) R,  R = sum_{M=J}^{I-1} A_IM T_MJ,  T_JJ = I + To_JJ.
+    // 16x16x16 products on v_mfma_f32_16x16x4f32 with the k index permuted so
+    // that at step kk lane group g supplies k = 4g + kk: the A operand of the
+    // four steps is one float4 of row m16, and a 16x16 block held in C layout
+    // (lane (g, m16) has rows 4g..4g+3 of column m16) is directly the B
+    // operand of the four steps.
+    auto mul = [&](f32x4 acc, const float* X, const f32x4& yb) __attribute__((always_inline)) {
+      const f32x4 xa = *reinterpret_cast<const f32x4*>(X + m16 * 16 + 4 * g4);
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int s = ks * 32 + slot_idx(g4, e);
-      f[e] = sT[t * kC + s] * fac[s];
+      for (int kk = 0; kk < 4; ++kk) acc = __builtin_amdgcn_mfma_f32_16x16x4f32(xa[kk], yb[kk], acc, 0, 0, 0);
+      return acc;
+    };
+    auto cblock = [&](const float* Y) __attribute__((always_inline)) {   // C layout of a block
+      f32x4 r;
+#pragma unroll
+      for (int j = 0; j < 4; ++j) r[j] = Y[(4 * g4 + j) * 16 + m16];
+      return r;
+    };
+    for (int d = 1; d < 4; ++d) {
+      if (w4 < 4 - d) {
+        const int J = w4, I = J + d;
+        f32x4 r = cblock(sA + tri(I, J) * 256);                             // A_IJ (identity part of T_JJ)
+        for (int M = J; M < I; ++M) r = mul(r, sA + tri(I, M) * 256, cblock(sT + tri(M, J) * 256));
+        const f32x4 tr = mul(r, sT + tri(I, I) * 256, r);                   // R + To_II R
+#pragma unroll
+        for (int jj = 0; jj < 4; ++jj) sT[tri(I, J) * 256 + (4 * g4 + jj) * 16 + m16] = -tr[jj];
+      }
+      __syncthreads();
     }
-    const u32x4 w = {pack_bf16x2(f[0], f[1]), pack_bf16x2(f[2], f[3]), pack_bf16x2(f[4], f[5]), pack_bf16x2(f[6], f[7])};
+    // ---- 7. To as a hi + lo pair in register order -------------------------------
 #pragma unroll
-    for (int e = 0; e < 8; ++e) r[e] = f[e] - __uint_as_float((e & 1) ? (w[e >> 1] & 0xffff0000u) : (w[e >> 1] << 16));
-    const u32x4 wl = {pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3]), pack_bf16x2(r[4], r[5]), pack_bf16x2(r[6], r[7])};
-    hi = as_bf16x8(w);
-    lo = as_bf16x8(wl);
-  };
-  auto b_operand = [&](const unsigned char* tile, bool trswz, int ks, int dt) __attribute__((always_inline)) {
-    const int d = dt * 16 + 4 * (m16 & 3);
-    const int r0 = ks * 32 + 4 * g4 + (m16 >> 2), r1 = r0 + 16;
-    const int z0 = trswz ? swz_tr(r0) : swz_rows(r0), z1 = trswz ? swz_tr(r1) : swz_rows(r1);
-    const u32x2 lo = ds_read_tr4(tile + r0 * RB + (((d >> 3) ^ z0) << 4) + ((d & 7) << 1));
-    const u32x2 hi = ds_read_tr4(tile + r1 * RB + (((d >> 3) ^ z1) << 4) + ((d & 7) << 1));
-    const u32x4 w = {lo[0], lo[1], hi[0], hi[1]};
-    return as_bf16x8(w);
-  };
-  {
-    bf16x8_t au[2], aul[2];
+    for (int ks = 0; ks < 2; ++ks) {
+      if (live && ks <= (w4 >> 1)) {
+        float f[8];
 #pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-      if (ks < nks) a_operand(ks, sBeta, au[ks], aul[ks]);
-    float* Uout = reinterpret_cast<float*>(rec + R::kU);
+        for (int h = 0; h < 2; ++h) {
+          const int J = 2 * ks + h;
+          const f32x4 x = *reinterpret_cast<const f32x4*>(sT + tri(w4, min(J, w4)) * 256 + m16 * 16 + 4 * g4);
 #pragma unroll
-    for (int dt = 0; dt < DV / 16; ++dt) {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < 2; ++ks)
-        if (ks < nks) {
-          const bf16x8_t vb = b_operand(sV, true, ks, dt);
-          acc = mfma16x16x32(au[ks], vb, acc);
-          acc = mfma16x16x32(aul[ks], vb, acc);
-          if constexpr (kLo) acc = mfma16x16x32(au[ks], b_operand(sQA, true, ks, dt), acc);
+          for (int j = 0; j < 4; ++j) f[4 * h + j] = J <= w4 ? x[j] : 0.f;
         }
-      // diagonal term: one transposing read gives V[ti*16 + 4*g4 + j][dt*16 + m16], j = 0..3
-      const int vr = ti * 16 + 4 * g4 + (m16 >> 2), vd = dt * 16 + 4 * (m16 & 3);
-      const int voff = vr * RB + (((vd >> 3) ^ swz_tr(vr)) << 4) + ((vd & 7) << 1);
-      const u32x2 vv = ds_read_tr4(sV + voff);
-      u32x2 vl = {0u, 0u};
-      if constexpr (kLo) vl = ds_read_tr4(sQA + voff);
-      const f32x4 bt = v4(sBeta, ti * 16 + g4 * 4);
-      f32x4 u;
-#pragma unroll
-      for (int j = 0; j < 4; ++j) {
-        float vf = __uint_as_float((j & 1) ? (vv[j >> 1] & 0xffff0000u) : (vv[j >> 1] << 16));
-        if constexpr (kLo) vf += __uint_as_float((j & 1) ? (vl[j >> 1] & 0xffff0000u) : (vl[j >> 1] << 16));
-        u[j] = acc[j] + bt[j] * vf;
-      }
-      __builtin_nontemporal_store(u, reinterpret_cast<f32x4*>(&Uout[((dt * 4 + ti) * 64 + lane) * 4]));
-    }
-  }
-  if constexpr (kLo) {
-    __syncthreads();                        // every wave is done with V
-    put_rows(sVW, false, kl1);              // K residual again (its first copy was overwritten by To)
-    __syncthreads();
-  }
-  // W^T (operands swapped: A = K^T by transposing reads, B = (To diag(sw))^T):
-  // the C layout gives lane (g4, m16) W[t = 16*tile + m16][d = 16*dt + 4*g4 + j],
-  // and d tiles 2*ks, 2*ks+1 together are its register-order slot of k-step ks.
-  {
-    const int t = ti * 16 + m16;
-    bf16x8_t bw[2], bwl[2];
-#pragma unroll
-    for (int ks = 0; ks < 2; ++ks)
-      if (ks < nks) a_operand(ks, sSw, bw[ks], bwl[ks]);
-    const float swt = sSw[t];
-    u32x4* Wout = reinterpret_cast<u32x4*>(rec + R::kW);
-    u32x4* WLout = reinterpret_cast<u32x4*>(rec + R::kWLo);
-#pragma unroll
-    for (int kso = 0; kso < DK / 32; ++kso) {
-      float wv[8];
-#pragma unroll
-      for (int h = 0; h < 2; ++h) {
-        const int dt = 2 * kso + h;
-        f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-        for (int ks = 0; ks < 2; ++ks)
-          if (ks < nks) {
-            const bf16x8_t kb = b_operand(sK, false, ks, dt);
-            acc = mfma16x16x32(kb, bw[ks], acc);
-            acc = mfma16x16x32(kb, bwl[ks], acc);
-            if constexpr (kLo) acc = mfma16x16x32(b_operand(sVW, false, ks, dt), bw[ks], acc);
-          }
-        const int d = dt * 16 + 4 * g4;
-        const int koff = t * RB + (((d >> 3) ^ swz_rows(t)) << 4) + ((d & 7) << 1);
-        const u32x2 kk = *reinterpret_cast<const u32x2*>(sK + koff);
-        u32x2 kl = {0u, 0u};
-        if constexpr (kLo) kl = *reinterpret_cast<const u32x2*>(sVW + koff);
-#pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          float kf = __uint_as_float((j & 1) ? (kk[j >> 1] & 0xffff0000u) : (kk[j >> 1] << 16));
-          if constexpr (kLo) kf += __uint_as_float((j & 1) ? (kl[j >> 1] & 0xffff0000u) : (kl[j >> 1] << 16));
-          wv[4 * h + j] = acc[j] + swt * kf;
-        }
-      }
-      const u32x4 wh = {pack_bf16x2(wv[0], wv[1]), pack_bf16x2(wv[2], wv[3]), pack_bf16x2(wv[4], wv[5]),
-                        pack_bf16x2(wv[6], wv[7])};
-      float wr[8];
-#pragma unroll
-      for (int e = 0; e < 8; ++e) wr[e] = wv[e] - __uint_as_float((e & 1) ? (wh[e >> 1] & 0xffff0000u) : (wh[e >> 1] << 16));
-      __builtin_nontemporal_store(wh, &Wout[(ti * 4 + kso) * 64 + lane]);
-      __builtin_nontemporal_store(u32x4{pack_bf16x2(wr[0], wr[1]), pack_bf16x2(wr[2], wr[3]),
-                                                pack_bf16x2(wr[4], wr[5]), pack_bf16x2(wr[6], wr[7])}, &WLout[(ti * 4 + kso) * 64 + lane]);
-    }
-  }
-  // ---- 6. K^T in slot order over tokens, straight from transposing reads --------
-  if (key_writer) {
-    bf16* Ktout = reinterpret_cast<bf16*>(krec + RK::kKt);
-    // 2 token k-steps x DK/16 key tiles = 16 jobs, 4 per wave
-#pragma unroll
-    for (int i = 0; i < 2 * (DK / 16) / 4; ++i) {
-      const int job = wave * (2 * (DK / 16) / 4) + i;
-      const int ks = job & 1, dt = job >> 1;
-      const bf16x8_t op = b_operand(sK, false, ks, dt);   // K[tokens in slot order][dt*16 + m16]
-      __builtin_nontemporal_store(__builtin_bit_cast(u32x4, op), reinterpret_cast<u32x4*>(&Ktout[((dt * 2 + ks) * 64 + lane) * 8]));
-      if constexpr (kLo) {
-        const bf16x8_t ol = b_operand(sVW, false, ks, dt);
-        __builtin_nontemporal_store(__builtin_bit_cast(u32x4, ol),
-                                    reinterpret_cast<u32x4*>(krec + RK::kKtLo + ((dt * 2 + ks) * 64 + lane) * 16));
+        u32x4 hi, lo;
+        split8(f, hi, lo);
+        __builtin_nontemporal_store(hi, reinterpret_cast<u32x4*>(rec + R::kT) + (w4 * 2 + ks) * 64 + lane);
+        __builtin_nontemporal_store(lo, reinterpret_cast<u32x4*>(rec + R::kTLo) + (w4 * 2 + ks) * 64 + lane);
       }
     }
-  }
-  // ---- 7. row factors --------------------------------------------------------
-  float* F = reinterpret_cast<float*>(rec + R::kF);
-  if (tid < kC) {
-    const float Glast = sGn[n - 1];
-    F[tid] = (tid < n) ? expf(sGn[tid]) * sIq[tid] : 0.f;            // fq
-    F[kC + tid] = (tid < n) ? expf(Glast - sGn[tid]) * sIk[tid] : 0.f;  // fk
-    if (tid == 0) F[2 * kC] = expf(Glast);                          // gamma
+    if ((pass + 1) * GP < G) {
+      __syncthreads();   // the gates and A of this pass are no longer read
+      gates(pass + 1);
+      __syncthreads();
+    }
   }
 }
 
 // ---------------------------------------------------------------------------
-// Per-chunk operands in registers (loaded two chunks ahead), by wave role.
+// Per-chunk operands in registers, by wave role.
 struct StateOps {
-  u32x4 w[4];        // W rows of token tile w4, k-steps 0..3 (slot order)
-  u32x4 wl[4];       // residual of W
-  u32x4 kt[2][2];    // K^T rows [key tile][token k-step]
-  f32x4 u;           // U (C layout)
-  f32x4 fk;          // fk of the 4 rows this lane holds
-  float gam;
+  u32x4 th[2], tl[2];    // To rows of token tile w4, token k-steps 0..1, and their residual
 };
+template <int NT, int RAW>
 struct OutOps {
   u32x4 q[4];        // Q rows of token tile w4, k-steps 0..3 (slot order)
   u32x4 p[2];        // P rows, token k-steps 0..1
-  f32x4 fq;
+  u32x2 v[RAW];      // V input rows (NT = 1: 4 columns, else this lane's NT)
 };
 
-// One workgroup = 8 waves on one (16-column slab, value head, sequence).
-// Waves 0-3 ("state" waves) carry the recurrence: each holds 32 key rows
-// of the slab's state and, per chunk, computes D = U - W S for token tile
-// w4, publishes D, then S = gamma S + K^T (fk D) for its key rows and
-// publishes S. Waves 4-7 ("output" waves) compute O = fq (Q S) + P D for
-// token tile w4 and store it. With two waves per SIMD the output path runs
-// beside the state path; the chunk's two barriers order both:
-//   A: state: W S, D, publish D        | output: Q S (S of this chunk)
-//   B: state: K^T (fk D), publish S'   | output: + P D, store
-template <int DK, int DV, bool kLo>
-__global__ __launch_bounds__(2 * kThreads, 1) void deltanet_chunk_scan_kernel(
-    const bf16* __restrict__ q, const unsigned char* __restrict__ ws, float* __restrict__ state,
+// One workgroup = 8 waves on NT 16-column tiles of one (value head, sequence).
+// Waves 0-3 ("state" waves) carry the recurrence: each holds 32 key rows of
+// the slab's state. Waves 4-7 ("output" waves) form the outputs of token tile
+// w4, V of the next chunk, and the DMAs that bring later chunks' K tiles.
+// With two waves per SIMD the output path runs beside the state path; three
+// barriers per chunk order both:
+//   A: state: R = beta V - sw (K S), publish R       | output: Q S
+//   B: state: D = R + To R, publish D and fk D       | output: V of the next chunk
+//   C: state: S' = gamma S + K^T (fk D), publish S'  | output: + P D, store
+// K tiles and register operands run NS - 1 chunks ahead.
+// Bound by the chunk's dependent chain (NT = 1: 62 of the scan's 85 us remain
+// with every load, DMA and V row taken out), then by its ~90 vector memory
+// instructions and the LDS traffic of the exchanges. Hence: row factors by DMA
+// instead of one load per wave and factor, V input in 4 loads of 8 bytes, not
+// 7 of 2 (103 -> 97 us together with it), and with one column tile the DMAs and
+// V on four helper waves (97 -> 89) whose DMAs follow V, since the wait the
+// compiler places for V's rows would cover them.
+template <bool kLo, int NT>
+__global__ __launch_bounds__(scan_threads(NT), 1) void deltanet_chunk_scan_kernel(
+    const bf16* __restrict__ v, ConvIn cv, const unsigned char* __restrict__ ws, float* __restrict__ state,
     bf16* __restrict__ out, int T, int Hk, int Hv, float scale) {
-  using R = ChunkRec<DK, DV>;
-  using RK = KeyRec<DK, kLo>;
-  static_assert(DK == 4 * 32, "the four state waves own 32 key rows each");
+  using R = ChunkRec;
+  using RK = KeyRec<kLo>;
+  constexpr int NS = NT <= 2 ? 3 : 2;            // chunks in flight (LDS stages, register sets)
+  constexpr int kSlabs = kD / (16 * NT);
+  // V input rows per lane: with one column tile a lane forms four columns of
+  // one token, else the four tokens of its C-layout registers (conv: + 3 rows)
+  constexpr int RAW = NT == 1 ? (kLo ? 4 : 1) : (kLo ? 7 : 4);
+  constexpr int kDma = (kLo ? 2 : 1) * kTile / 1024 / 4;   // DMA instructions per output wave and chunk
   // XCD-aware placement: workgroups are dispatched round-robin over the 8
-  // XCDs, so linear id i runs on XCD i % 8. All DV/16 slabs of one head are
-  // put on the same XCD, where they share the head's chunk records in L2
-  // (otherwise every XCD fetches them from HBM), and each XCD takes a
-  // contiguous range of heads, so that the value heads of a key head also
-  // share its key-head records there.
-  constexpr int kSlabs = DV / 16;
-  const int nhead = static_cast<int>(gridDim.y * gridDim.z);
-  const int lin = blockIdx.x + kSlabs * (blockIdx.y + static_cast<int>(gridDim.y) * blockIdx.z);
-  int slab = blockIdx.x, headlin = blockIdx.y + static_cast<int>(gridDim.y) * blockIdx.z;
-  if (kSlabs == kNumXcd && nhead % kNumXcd == 0) {
-    const int xcd = lin % kNumXcd, i = lin / kNumXcd;
-    slab = i % kSlabs;
-    headlin = xcd * (nhead / kNumXcd) + i / kSlabs;
-  }
+  // XCDs, so linear id i runs on XCD i % 8. The slabs of a head are put on
+  // the same XCD, where they share the head's chunk records in L2 (otherwise
+  // every XCD fetches them from HBM), and each XCD takes a contiguous range
+  // of heads, so that the value heads of a key head also share its key-head
+  // records there.
+  const int nwg = static_cast<int>(gridDim.x * gridDim.y * gridDim.z);
+  int lin = blockIdx.x + kSlabs * (blockIdx.y + static_cast<int>(gridDim.y) * blockIdx.z);
+  if (nwg % kNumXcd == 0) lin = (lin % kNumXcd) * (nwg / kNumXcd) + lin / kNumXcd;
+  const int slab = lin % kSlabs, headlin = lin / kSlabs;
   const int hv = headlin % Hv, b = headlin / Hv;
   const int nch = (T + kC - 1) / kC;
   const int tid = threadIdx.x, lane = tid & 63;
   const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
   const int w4 = wave & 3;
   const int m16 = lane & 15, g4 = lane >> 4;
-  const int col = slab * 16 + m16;
+  // Column m16 of the NT tiles is column m16 * NT + nt of the slab, so that a
+  // lane's columns are contiguous in the state, the V rows and the outputs.
+  const int col = (slab * 16 + m16) * NT;
 
-  __shared__ u32x4 sS[4][64];            // S B-operands, one per 32-row k-step
-  __shared__ u32x4 sSl[4][64];           // residual of S
-  __shared__ u32x2 sD[2][2][64];         // D (bf16) B-operands: [k-step][half][lane]
-  __shared__ u32x2 sDh[2][2][64];        // (fk D) hi
-  __shared__ u32x2 sDl[2][2][64];        // (fk D) lo
+  __shared__ __attribute__((aligned(1024))) unsigned char sK[NS][kTile];
+  __shared__ __attribute__((aligned(1024))) unsigned char sKl[kLo ? NS : 1][kLo ? kTile : 16];
+  __shared__ u32x4 sS[NT][4][64];            // S B-operands, one per 32-row k-step
+  __shared__ u32x4 sSl[NT][4][64];           // residual of S
+  __shared__ u32x2 sRh[NT][2][2][64], sRl[NT][2][2][64];   // R hi, lo: [k-step][half][lane]
+  __shared__ u32x2 sD[NT][2][2][64];         // D (bf16)
+  __shared__ u32x2 sDh[NT][2][2][64], sDl[NT][2][2][64];   // (fk D) hi, lo
+  __shared__ __attribute__((aligned(256))) float sF[NS][5][kC];   // row factors of the record
+  // V rows. One column tile: [token][column], rows padded to 20 floats; else C
+  // layout. By chunk parity where the next chunk's V is formed in phase A.
+  constexpr int kVRow = 20;
+  __shared__ __attribute__((aligned(16))) float sV1[NT == 1 ? 2 : 1][NT == 1 ? kC * kVRow : 4];
+  __shared__ f32x4 sV[NT == 2 ? 2 : 1][NT == 1 ? 1 : NT][4][64];
 
   const unsigned char* recs = ws + (static_cast<size_t>(b) * Hv + hv) * nch * R::kBytes;
   auto rec_of = [&](int c) __attribute__((always_inline)) { return recs + static_cast<size_t>(c) * R::kBytes; };
   const unsigned char* krecs =
-      ws + key_rec_offset<DK, DV, kLo>(b, hv / (Hv / Hk), 0, static_cast<int>(gridDim.z), Hk, Hv, nch);
+      ws + key_rec_offset<kLo>(b, hv / (Hv / Hk), 0, static_cast<int>(gridDim.z), Hk, Hv, nch);
   auto krec_of = [&](int c) __attribute__((always_inline)) { return krecs + static_cast<size_t>(c) * RK::kBytes; };
 
   if (wave < 4) {
     // ------------------------------------------------------------ state waves
-    // Operands of a chunk in eight parts (0-3: W and W_lo of k-step p;
-    // 4-5: K^T of key tile p-4; 7: U and the factors; 6 is empty - the K^T
-    // residual of split inputs is loaded by its own chunk, half a chunk
-    // ahead of its use, which keeps that variant within the register file).
-    // The parts are issued one per MFMA group of an earlier chunk, in an
-    // order that differs between slabs (below).
-    auto load = [&](int c, StateOps& o, int part) __attribute__((always_inline)) {
+    auto load = [&](int c, StateOps& o) __attribute__((always_inline)) {
       const unsigned char* rec = rec_of(c);
-      if (part < 4) {
-        o.w[part] = reinterpret_cast<const u32x4*>(rec + R::kW)[(w4 * 4 + part) * 64 + lane];
-        o.wl[part] = reinterpret_cast<const u32x4*>(rec + R::kWLo)[(w4 * 4 + part) * 64 + lane];
-      } else if (part < 6) {
-        const int tt = part - 4;
-        const u32x4* Kt = reinterpret_cast<const u32x4*>(krec_of(c) + RK::kKt) + lane;
-#pragma unroll
-        for (int s2 = 0; s2 < 2; ++s2) o.kt[tt][s2] = Kt[((w4 * 2 + tt) * 2 + s2) * 64];
-      } else if (part == 6) {
-        // (the K^T residual of split inputs is loaded by the chunk itself)
-      } else {
-        o.u = *reinterpret_cast<const f32x4*>(rec + R::kU + ((slab * 4 + w4) * 64 + lane) * 16);
-        const float* F = reinterpret_cast<const float*>(rec + R::kF);
-        o.fk = *reinterpret_cast<const f32x4*>(F + kC + w4 * 16 + g4 * 4);
-        o.gam = F[2 * kC];
+      const u32x4* Th = reinterpret_cast<const u32x4*>(rec + R::kT) + w4 * 128 + lane;
+      const u32x4* Tl = reinterpret_cast<const u32x4*>(rec + R::kTLo) + w4 * 128 + lane;
+      o.th[0] = Th[0];
+      o.tl[0] = Tl[0];
+      if (w4 >= 2) {
+        o.th[1] = Th[64];
+        o.tl[1] = Tl[64];
       }
     };
-    // state slab in C layout: rows 32*w4 + 16*tt + 4*g4 + j, column col
-    float* Sg = state + (static_cast<size_t>(b) * Hv + hv) * DK * DV;
-    float s_reg[2][4];
+    auto factor = [&](const float (&f)[5][kC], int which) __attribute__((always_inline)) {
+      return *reinterpret_cast<const f32x4*>(&f[which][w4 * 16 + g4 * 4]);
+    };
+    // state slab in C layout: rows 32*w4 + 16*tt + 4*g4 + j, column col + nt
+    float* Sg = state + (static_cast<size_t>(b) * Hv + hv) * kD * kD + static_cast<size_t>(w4 * 32 + g4 * 4) * kD + col;
+    float s_reg[NT][8];
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
+    for (int e = 0; e < 8; ++e)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) s_reg[tt][j] = Sg[static_cast<size_t>(w4 * 32 + tt * 16 + g4 * 4 + j) * DV + col];
+      for (int nt = 0; nt < NT; ++nt) s_reg[nt][e] = Sg[((e >> 2) * 16 + (e & 3)) * kD + nt];
+    u32x4 s_hi[NT], s_lo[NT];   // this wave's own k-step of the S operand
     auto publish_state = [&]() __attribute__((always_inline)) {
-      const u32x4 w = {pack_bf16x2(s_reg[0][0], s_reg[0][1]), pack_bf16x2(s_reg[0][2], s_reg[0][3]),
-                       pack_bf16x2(s_reg[1][0], s_reg[1][1]), pack_bf16x2(s_reg[1][2], s_reg[1][3])};
-      float r[8];
 #pragma unroll
-      for (int e = 0; e < 8; ++e)
-        r[e] = s_reg[e >> 2][e & 3] - __uint_as_float((e & 1) ? (w[e >> 1] & 0xffff0000u) : (w[e >> 1] << 16));
-      sS[w4][lane] = w;
-      sSl[w4][lane] = u32x4{pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3]), pack_bf16x2(r[4], r[5]),
-                            pack_bf16x2(r[6], r[7])};
+      for (int nt = 0; nt < NT; ++nt) {
+        split8(s_reg[nt], s_hi[nt], s_lo[nt]);
+        sS[nt][w4][lane] = s_hi[nt];
+        sSl[nt][w4][lane] = s_lo[nt];
+      }
     };
+    const int s2w = w4 >> 1, halfw = w4 & 1;
     // `active` is uniform; an inactive chunk (past the last one, padding the
-    // three-chunk rotation) computes on repeated operands but keeps its state
-    // (a select, so the chunk body stays one basic block for the schedule).
-    // ROT: this slab's rotation of the load order (see the loop below).
-    auto chunk = [&](bool active, const StateOps& o, int cc, int cn, StateOps& on, auto rot_c) __attribute__((always_inline)) {
-      // split inputs: the K^T residual of this chunk, loaded now (half a
-      // chunk ahead of its use) instead of in the rotating sets
-      u32x4 ktl[2][2];
-      if constexpr (kLo) {
-        const u32x4* Ktl = reinterpret_cast<const u32x4*>(krec_of(min(cc, nch - 1)) + RK::kKtLo) + lane;
+    // rotation) computes on repeated operands but keeps its state (a select,
+    // so the chunk body stays one basic block for the schedule).
+    // K rows of token tile w4, read a phase ahead; k-step (w4 + i) % 4 at i, so
+    // that the first products take the wave's own state rows from registers
+    bf16x8_t kh[4], kl[4];
+    auto read_k = [&](const unsigned char* kt, const unsigned char* klt) __attribute__((always_inline)) {
 #pragma unroll
-        for (int tt = 0; tt < 2; ++tt)
-#pragma unroll
-          for (int s2 = 0; s2 < 2; ++s2) ktl[tt][s2] = Ktl[((w4 * 2 + tt) * 2 + s2) * 64];
+      for (int i = 0; i < 4; ++i) {
+        kh[i] = row_operand<kLo>(kt, (w4 + i) & 3, w4 * 16 + m16, g4);
+        if constexpr (kLo) kl[i] = row_operand<kLo>(klt, (w4 + i) & 3, w4 * 16 + m16, g4);
       }
-      constexpr int ROT = decltype(rot_c)::value;
-      // A: D = U - W S (hi*hi + hi*lo + lo*hi), published as bf16 and as
-      //    hi/lo bf16 of fk D
-      {
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
+    };
+    auto chunk = [&](auto pos, bool active, int c, const StateOps& o, StateOps& on) __attribute__((always_inline)) {
+      constexpr int st = decltype(pos)::value, stn = (st + 1) % NS;
+      // A: R = beta V - sw (K S) of token tile w4
+      const f32x4 beta = factor(sF[st], 2), sw = factor(sF[st], 3), fk = factor(sF[st], 1);
+      const float gam = sF[st][4][lane];
+      f32x4 r[NT];
+      bf16x8_t kth[2][2], ktl[2][2];
 #pragma unroll
-      for (int ks = 0; ks < DK / 32; ++ks) {
-        const bf16x8_t sh = as_bf16x8(sS[ks][lane]);
-        acc = mfma16x16x32(as_bf16x8(o.w[ks]), sh, acc);
-        acc = mfma16x16x32(as_bf16x8(o.w[ks]), as_bf16x8(sSl[ks][lane]), acc);
-        acc = mfma16x16x32(as_bf16x8(o.wl[ks]), sh, acc);
-        load(cn, on, (ks + 2 * ROT) & 7);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-      {
-        float dval[4], dsc[4], lo[4];
+      for (int nt = 0; nt < NT; ++nt) {
+        f32x4 acc = {0.f, 0.f, 0.f, 0.f}, acl = {0.f, 0.f, 0.f, 0.f}, acm = {0.f, 0.f, 0.f, 0.f};
 #pragma unroll
-        for (int j = 0; j < 4; ++j) {
-          dval[j] = o.u[j] - acc[j];
-          dsc[j] = o.fk[j] * dval[j];
+        for (int i = 0; i < 4; ++i) {
+          const int ks = (w4 + i) & 3;
+          const bf16x8_t sh = as_bf16x8(i == 0 ? s_hi[nt] : sS[nt][ks][lane]);
+          const bf16x8_t sl = as_bf16x8(i == 0 ? s_lo[nt] : sSl[nt][ks][lane]);
+          acc = mfma16x16x32(kh[i], sh, acc);
+          acl = mfma16x16x32(kh[i], sl, acl);
+          if constexpr (kLo) acm = mfma16x16x32(kl[i], sh, acm);
         }
-        const int s2 = w4 >> 1, half = w4 & 1;
-        sD[s2][half][lane] = u32x2{pack_bf16x2(dval[0], dval[1]), pack_bf16x2(dval[2], dval[3])};
-        const u32x2 hp = {pack_bf16x2(dsc[0], dsc[1]), pack_bf16x2(dsc[2], dsc[3])};
+        if (nt == 0) {   // the K^T operands of phase C, read under the arithmetic
 #pragma unroll
-        for (int j = 0; j < 4; ++j)
-          lo[j] = dsc[j] - __uint_as_float((j & 1) ? (hp[j >> 1] & 0xffff0000u) : (hp[j >> 1] << 16));
-        sDh[s2][half][lane] = hp;
-        sDl[s2][half][lane] = u32x2{pack_bf16x2(lo[0], lo[1]), pack_bf16x2(lo[2], lo[3])};
-      }
+          for (int tt = 0; tt < 2; ++tt)
+#pragma unroll
+            for (int s2 = 0; s2 < 2; ++s2) {
+              kth[tt][s2] = tr_operand<kLo>(sK[st], s2, w4 * 2 + tt, m16, g4);
+              if constexpr (kLo) ktl[tt][s2] = tr_operand<kLo>(sKl[st], s2, w4 * 2 + tt, m16, g4);
+            }
+        }
+        if constexpr (kLo) acl += acm;
+        f32x4 vr;
+        if constexpr (NT == 1) {
+#pragma unroll
+          for (int j = 0; j < 4; ++j) vr[j] = sV1[c & 1][(w4 * 16 + g4 * 4 + j) * kVRow + m16];
+        } else {
+          vr = sV[NT == 2 ? c & 1 : 0][nt][w4][lane];
+        }
+        r[nt] = beta * vr - sw * (acc + acl);
+        u32x2 hi, lo;
+        split4(r[nt], hi, lo);
+        sRh[nt][s2w][halfw][lane] = hi;
+        sRl[nt][s2w][halfw][lane] = lo;
       }
       phase_barrier();
-      // B: S = gamma S + K^T (fk D) for the key rows of this wave
-      {
-      bf16x8_t dh[2], dl[2];
+      // B: D = R + To R
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2) {
-        dh[s2] = cat8x2(sDh[s2][0][lane], sDh[s2][1][lane]);
-        dl[s2] = cat8x2(sDl[s2][0][lane], sDl[s2][1][lane]);
+      for (int nt = 0; nt < NT; ++nt) {
+        f32x4 d = r[nt], dl = {0.f, 0.f, 0.f, 0.f}, dm = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2)
+          if (s2 <= s2w) {
+            const bf16x8_t rh = cat8x2(sRh[nt][s2][0][lane], sRh[nt][s2][1][lane]);
+            const bf16x8_t rl = cat8x2(sRl[nt][s2][0][lane], sRl[nt][s2][1][lane]);
+            d = mfma16x16x32(as_bf16x8(o.th[s2]), rh, d);
+            dl = mfma16x16x32(as_bf16x8(o.th[s2]), rl, dl);
+            dm = mfma16x16x32(as_bf16x8(o.tl[s2]), rh, dm);
+          }
+        d += dl + dm;
+        sD[nt][s2w][halfw][lane] = u32x2{pack_bf16x2(d[0], d[1]), pack_bf16x2(d[2], d[3])};
+        u32x2 hi, lo;
+        split4(fk * d, hi, lo);
+        sDh[nt][s2w][halfw][lane] = hi;
+        sDl[nt][s2w][halfw][lane] = lo;
       }
+      phase_barrier();
+      // C: S = gamma S + K^T (fk D) for the key rows of this wave
 #pragma unroll
-      for (int tt = 0; tt < 2; ++tt) {
-        f32x4 a2 = {0.f, 0.f, 0.f, 0.f};
+      for (int nt = 0; nt < NT; ++nt) {
+        f32x4 a2[2] = {{0.f, 0.f, 0.f, 0.f}, {0.f, 0.f, 0.f, 0.f}};
 #pragma unroll
         for (int s2 = 0; s2 < 2; ++s2) {
-          const bf16x8_t aK = as_bf16x8(o.kt[tt][s2]);
-          a2 = mfma16x16x32(aK, dh[s2], a2);
-          a2 = mfma16x16x32(aK, dl[s2], a2);
-          if constexpr (kLo) a2 = mfma16x16x32(as_bf16x8(ktl[tt][s2]), dh[s2], a2);
-          load(cn, on, (4 + 2 * tt + s2 + 2 * ROT) & 7);
-          __builtin_amdgcn_sched_barrier(0);
-        }
+          const bf16x8_t dh = cat8x2(sDh[nt][s2][0][lane], sDh[nt][s2][1][lane]);
+          const bf16x8_t dl = cat8x2(sDl[nt][s2][0][lane], sDl[nt][s2][1][lane]);
 #pragma unroll
-        for (int j = 0; j < 4; ++j) s_reg[tt][j] = active ? o.gam * s_reg[tt][j] + a2[j] : s_reg[tt][j];
+          for (int tt = 0; tt < 2; ++tt) {
+            a2[tt] = mfma16x16x32(kth[tt][s2], dh, a2[tt]);
+            a2[tt] = mfma16x16x32(kth[tt][s2], dl, a2[tt]);
+            if constexpr (kLo) a2[tt] = mfma16x16x32(ktl[tt][s2], dh, a2[tt]);
+          }
+        }
+        if (NS == 3 && nt == 0) read_k(sK[stn], sKl[kLo ? stn : 0]);   // of the next chunk (landed since barrier 2)
+#pragma unroll
+        for (int e = 0; e < 8; ++e)
+          s_reg[nt][e] = active ? gam * s_reg[nt][e] + a2[e >> 2][e & 3] : s_reg[nt][e];
       }
       publish_state();
-      }
+      load(min(c + NS - 1, nch - 1), on);
       phase_barrier();
+      if constexpr (NS == 2) read_k(sK[stn], sKl[kLo ? stn : 0]);
     };
     publish_state();
-    // Three operand sets rotate; loads are unconditional (clamped to the
-    // last chunk) so that the compiler's wait counts stay exact.
-    // The slabs of a head read the same chunk records at about the same
-    // time; each group of slabs issues the parts in a different order, so
-    // that their requests meet fewer times on one L2 channel (config 4:
-    // 171 -> 160 us; layer prefill 271 -> 258 us).
-    auto run = [&](auto rot_c) __attribute__((always_inline)) {
-      StateOps o0, o1, o2;
+    // Register sets rotate; loads are unconditional (clamped to the last
+    // chunk) so that the compiler's wait counts stay exact.
+    StateOps o[NS];
 #pragma unroll
-      for (int part = 0; part < 8; ++part) load(0, o0, part);
-#pragma unroll
-      for (int part = 0; part < 8; ++part) load(min(1, nch - 1), o1, part);
-      __syncthreads();
-      for (int c = 0; c < nch; c += 3) {
-        chunk(true, o0, c, min(c + 2, nch - 1), o2, rot_c);
-        chunk(c + 1 < nch, o1, c + 1, min(c + 3, nch - 1), o0, rot_c);
-        chunk(c + 2 < nch, o2, c + 2, min(c + 4, nch - 1), o1, rot_c);
-      }
-    };
-    switch (slab & 3) {
-      case 0: run(std::integral_constant<int, 0>{}); break;
-      case 1: run(std::integral_constant<int, 1>{}); break;
-      case 2: run(std::integral_constant<int, 2>{}); break;
-      default: run(std::integral_constant<int, 3>{}); break;
+    for (int i = 0; i < NS - 1; ++i) load(min(i, nch - 1), o[i]);
+    __syncthreads();
+    read_k(sK[0], sKl[0]);
+    for (int c = 0; c < nch; c += NS) {
+      chunk(std::integral_constant<int, 0>{}, true, c, o[0], o[NS - 1]);
+      chunk(std::integral_constant<int, 1>{}, c + 1 < nch, c + 1, o[1], o[0]);
+      if constexpr (NS == 3) chunk(std::integral_constant<int, NS - 1>{}, c + 2 < nch, c + 2, o[NS - 1], o[1]);
     }
 #pragma unroll
-    for (int tt = 0; tt < 2; ++tt)
+    for (int e = 0; e < 8; ++e)
 #pragma unroll
-      for (int j = 0; j < 4; ++j) Sg[static_cast<size_t>(w4 * 32 + tt * 16 + g4 * 4 + j) * DV + col] = s_reg[tt][j];
+      for (int nt = 0; nt < NT; ++nt) Sg[((e >> 2) * 16 + (e & 3)) * kD + nt] = s_reg[nt][e];
   } else {
-    // ----------------------------------------------------------- output waves
-    // parts 0-3: Q of k-step p; 4: P and fq (interleaved as in the state waves)
-    auto load = [&](int c, OutOps& o, int part) __attribute__((always_inline)) {
-      const unsigned char* rec = rec_of(c);
-      if (part < 4) {
-        o.q[part] = reinterpret_cast<const u32x4*>(krec_of(c) + RK::kQ)[(w4 * 4 + part) * 64 + lane];
-      } else {
-        const u32x4* P = reinterpret_cast<const u32x4*>(rec + R::kP) + w4 * 2 * 64 + lane;
-        o.p[0] = P[0];
-        o.p[1] = P[64];
-        o.fq = *reinterpret_cast<const f32x4*>(reinterpret_cast<const float*>(rec + R::kF) + w4 * 16 + g4 * 4);
+    // ------------------------------------------------- output and helper waves
+    constexpr bool kHelp = NT == 1;
+    const bool outw = wave < 8;   // else helper
+    using Ops = OutOps<NT, RAW>;
+    const int trow = w4 * 16 + g4 * 4;             // first of this lane's 4 token rows
+    // first token and V channel this lane forms, and its number of channels
+    const int vtok = NT == 1 ? w4 * 16 + (lane >> 2) : trow;
+    const int vch = (kLo ? 2 * Hk * kD : 0) + hv * kD + (NT == 1 ? slab * 16 + (lane & 3) * 4 : col);
+    constexpr int NV = NT == 1 ? 4 : NT;
+    float cw[NV][4];                               // conv taps
+    if constexpr (kLo) {
+#pragma unroll
+      for (int e = 0; e < NV; ++e) {
+        const u32x2 w = *reinterpret_cast<const u32x2*>(cv.w + static_cast<size_t>(vch + e) * 4);
+#pragma unroll
+        for (int i = 0; i < 4; ++i) cw[e][i] = bf_at(w, i);
       }
+    }
+    auto load_v = [&](int c, Ops& o) __attribute__((always_inline)) {
+      // V input rows, through a resource that ends at the chunk's last token
+      // (rows past it read as zeros). The rows a lane needs start at its first
+      // token, less the conv's three (`lead` of which lie before the chunk; in
+      // the first chunk those come from the ring, in form_v).
+      const int t0 = c * kC, lead = kLo && c > 0 ? 3 : 0, back = kLo ? 3 : 0;
+      const int stride = kLo ? cv.stride : Hv * kD;
+      const bf16* base = (kLo ? cv.qkv : v) + (static_cast<size_t>(b) * T + t0 - lead) * stride;
+      const __amdgpu_buffer_rsrc_t rs = __builtin_amdgcn_make_buffer_rsrc(
+          const_cast<bf16*>(base), 0, (min(kC, T - t0) + lead) * stride * 2, kBufferRsrcWord3);
+#pragma unroll
+      for (int i = 0; i < RAW; ++i) {
+        const int at = (max(vtok - back + i + lead, 0) * stride + vch) * 2;
+        if constexpr (NT == 2) o.v[i][0] = __builtin_amdgcn_raw_buffer_load_b32(rs, at, 0, 0);
+        else o.v[i] = __builtin_bit_cast(u32x2, __builtin_amdgcn_raw_buffer_load_b64(rs, at, 0, 0));
+      }
+    };
+    auto load_qp = [&](int c, Ops& o) __attribute__((always_inline)) {
+      const unsigned char* rec = rec_of(c);
+      const u32x4* Q = reinterpret_cast<const u32x4*>(krec_of(c) + RK::kQ) + w4 * 256 + lane;
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) o.q[ks] = Q[ks * 64];
+      const u32x4* P = reinterpret_cast<const u32x4*>(rec + R::kP) + w4 * 128 + lane;
+      o.p[0] = P[0];
+      if (w4 >= 2) o.p[1] = P[64];
+    };
+    // V of chunk c (the layer: conv + SiLU of its raw rows), published for the
+    // state waves; `first`: chunk 0, whose first rows reach into the ring
+    auto form_v = [&](int c, const Ops& o, bool first) __attribute__((always_inline)) {
+      constexpr int TOK = NT == 1 ? 1 : 4;         // tokens per lane
+      float y[NV][TOK];
+#pragma unroll
+      for (int e = 0; e < NV; ++e) {
+        float x[RAW];
+#pragma unroll
+        for (int i = 0; i < RAW; ++i) x[i] = bf_at(o.v[i], e);
+        if constexpr (kLo) {
+          if (first && vtok < 3) {
+            const int head = ((cv.head % 3) + 3) % 3;
+#pragma unroll
+            for (int i = 0; i < 3; ++i)
+              if (vtok - 3 + i < 0)
+                x[i] = cv.ring[(static_cast<size_t>(b) * 3 + (head + vtok + i) % 3) * cv.ch + vch + e];
+          }
+#pragma unroll
+          for (int j = 0; j < TOK; ++j) {
+            float acc = x[j] * cw[e][0];
+            acc += x[j + 1] * cw[e][1];
+            acc += x[j + 2] * cw[e][2];
+            acc += x[j + 3] * cw[e][3];
+            const float sg = __builtin_amdgcn_rcpf(1.0f + __builtin_amdgcn_exp2f(-acc * kLog2e));
+            y[e][j] = (c * kC + vtok + j < T) ? acc * sg : 0.f;
+          }
+        } else {
+#pragma unroll
+          for (int j = 0; j < TOK; ++j) y[e][j] = x[j];
+        }
+      }
+      if constexpr (NT == 1) {
+        *reinterpret_cast<f32x4*>(&sV1[c & 1][vtok * kVRow + (lane & 3) * 4]) = f32x4{y[0][0], y[1][0], y[2][0], y[3][0]};
+      } else {
+#pragma unroll
+        for (int nt = 0; nt < NT; ++nt) sV[NT == 2 ? c & 1 : 0][nt][w4][lane] = f32x4{y[nt][0], y[nt][1], y[nt][2], y[nt][3]};
+      }
+    };
+    // K tile(s) and row factors of chunk c -> LDS stage, the wave's share of
+    // wave-contiguous KiB. (The DMA builtin makes the compiler wait for every load in flight
+    // before the next LDS read; the wrapper's DMAs are ordered by hand below.)
+    auto dma_k = [&](int c, unsigned char* kt, unsigned char* klt, float* ft) __attribute__((always_inline)) {
+      const u32x4 src = buffer_rsrc(krec_of(c), static_cast<int>(RK::kBytes));
+#pragma unroll
+      for (int i = 0; i < kTile / 1024 / 4; ++i) {
+        const int slot = (i * 4 + w4) * 1024;
+        dma16_to_lds(src, static_cast<int>(RK::kK) + slot + lane * 16, kt + slot);
+        if constexpr (kLo) dma16_to_lds(src, static_cast<int>(RK::kKLo) + slot + lane * 16, klt + slot);
+      }
+      const u32x4 fsrc = buffer_rsrc(rec_of(c), 5 * kC * 4);
+      if (w4 == 0) dma16_to_lds(fsrc, lane * 16, ft);
+      if (w4 == 1 && lane < 16) dma16_to_lds(fsrc, 1024 + lane * 16, ft + 256);
     };
     // Output rows go out through a buffer resource bounded at the chunk's
     // last token, so the stores need no per-row branch (rows past T drop).
-    const int rs2 = Hv * DV * 2;   // bytes per token row
-    const int lane_off = ((w4 * 16 + g4 * 4) * Hv + hv) * DV * 2 + col * 2;
-    auto chunk = [&](bool active, int c, const OutOps& o, int cn, OutOps& on, auto rot_c) __attribute__((always_inline)) {
-      constexpr int ROT = decltype(rot_c)::value;
-      // A: Q S with the state of this chunk
-      f32x4 acc = {0.f, 0.f, 0.f, 0.f};
-#pragma unroll
-      for (int ks = 0; ks < DK / 32; ++ks) {
-        const bf16x8_t sh = as_bf16x8(sS[ks][lane]);
-        acc = mfma16x16x32(as_bf16x8(o.q[ks]), sh, acc);
-        // split inputs: S as hi + lo (the residual of Q adds ~15% to the
-        // scan's operand bytes for no measurable gain: P carries it)
-        if constexpr (kLo) acc = mfma16x16x32(as_bf16x8(o.q[ks]), as_bf16x8(sSl[ks][lane]), acc);
-        load(cn, on, (ks + ROT) % 5);
-        __builtin_amdgcn_sched_barrier(0);
-      }
-#pragma unroll
-      for (int j = 0; j < 4; ++j) acc[j] *= o.fq[j];
+    const int rs2 = Hv * kD * 2;   // bytes per token row
+    const int lane_off = trow * rs2 + (hv * kD + col) * 2;
+    // Three stages: the K tile of chunk cn = c + 2 goes out, V of chunk c + 1 is
+    // formed. The K tile of chunk c + 1 must have landed: its DMAs were issued
+    // a chunk ago, and the vector memory operations since then (for an output
+    // wave also its stores, Q and P, at least one of it) may stay in flight.
+    // (V first: its wait for the rows, which the compiler places, would
+    // otherwise cover the DMAs just issued.)
+    auto supply = [&](int c, int cn, int nst, const Ops& ov, Ops& on) __attribute__((always_inline)) {
+      form_v(c + 1, ov, false);
+      load_v(cn, on);
+      dma_k(cn, sK[nst], sKl[kLo ? nst : 0], &sF[nst][0][0]);
+      __builtin_amdgcn_s_waitcnt(vmcnt_imm<(kHelp ? 0 : 4 + 4 + 1) + RAW + kDma>());
+    };
+    auto helper = [&](auto pos, int c, const Ops& ov, Ops& on) __attribute__((always_inline)) {
+      supply(c, min(c + NS - 1, nch - 1), (decltype(pos)::value + NS - 1) % NS, ov, on);
       phase_barrier();
-      // B: + P D, store (an inactive chunk's resource holds no bytes)
+      phase_barrier();
+      phase_barrier();
+    };
+    auto chunk = [&](auto pos, bool active, int c, const Ops& o, const Ops& ov, Ops& on) __attribute__((always_inline)) {
+      constexpr int cst = decltype(pos)::value;
+      constexpr int nst = (decltype(pos)::value + NS - 1) % NS;   // stage of chunk c + NS - 1 (free since chunk c - 1)
+      const int cn = min(c + NS - 1, nch - 1);
+      if constexpr (NS == 2) {
+        load_v(cn, on);
+        dma_k(cn, sK[nst], sKl[kLo ? nst : 0], &sF[nst][0][0]);
+        load_qp(cn, on);
+      }
+      f32x4 acc[NT];
+      auto q_s = [&]() __attribute__((always_inline)) {   // Q S with the state of this chunk
+        const f32x4 fq = *reinterpret_cast<const f32x4*>(&sF[cst][0][trow]);
 #pragma unroll
-      for (int s2 = 0; s2 < 2; ++s2)
-        if (s2 <= (w4 >> 1)) acc = mfma16x16x32(as_bf16x8(o.p[s2]), cat8x2(sD[s2][0][lane], sD[s2][1][lane]), acc);
-      load(cn, on, (4 + ROT) % 5);
+        for (int nt = 0; nt < NT; ++nt) {
+          acc[nt] = f32x4{0.f, 0.f, 0.f, 0.f};
+          f32x4 acl = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+          for (int ks = 0; ks < 4; ++ks) {
+            acc[nt] = mfma16x16x32(as_bf16x8(o.q[ks]), as_bf16x8(sS[nt][ks][lane]), acc[nt]);
+            // split inputs: S as hi + lo (the residual of Q adds ~15% to the
+            // scan's operand bytes for no measurable gain: P carries it)
+            if constexpr (kLo) acl = mfma16x16x32(as_bf16x8(o.q[ks]), as_bf16x8(sSl[nt][ks][lane]), acl);
+          }
+          if constexpr (kLo) acc[nt] += acl;
+          acc[nt] *= fq;
+        }
+      };
+      // A and B: Q S and the loads of a later chunk. Q S goes first with one
+      // column tile; with more, the state waves first have the LDS to themselves
+      // for their reads of S (4 tiles, 96 heads: 150 against 157 us a layer).
+      if constexpr (kHelp) q_s();
+      else if constexpr (NS == 3) supply(c, cn, nst, ov, on);
+      phase_barrier();
+      if constexpr (NS == 3) load_qp(cn, on);
+      if constexpr (!kHelp) q_s();
+      phase_barrier();
+      // C: + P D, store (an inactive chunk's resource holds no bytes)
       const int t0 = min(c, nch - 1) * kC;
       const __amdgpu_buffer_rsrc_t orsrc = __builtin_amdgcn_make_buffer_rsrc(
-          out + (static_cast<size_t>(b) * T + t0) * Hv * DV, 0, active ? min(kC, T - t0) * rs2 : 0, kBufferRsrcWord3);
+          out + (static_cast<size_t>(b) * T + t0) * Hv * kD, 0, active ? min(kC, T - t0) * rs2 : 0, kBufferRsrcWord3);
 #pragma unroll
-      for (int j = 0; j < 4; ++j)
-        __builtin_amdgcn_raw_buffer_store_b16(f2bf(scale * acc[j]), orsrc, lane_off + j * rs2, 0, 0);
+      for (int nt = 0; nt < NT; ++nt) {
+#pragma unroll
+        for (int s2 = 0; s2 < 2; ++s2)
+          if (s2 <= (w4 >> 1))
+            acc[nt] = mfma16x16x32(as_bf16x8(o.p[s2]), cat8x2(sD[nt][s2][0][lane], sD[nt][s2][1][lane]), acc[nt]);
+      }
+#pragma unroll
+      for (int j = 0; j < 4; ++j) {
+        const int at = lane_off + j * rs2;
+        if constexpr (NT == 1)
+          __builtin_amdgcn_raw_buffer_store_b16(static_cast<uint16_t>(pack_bf16x2(scale * acc[0][j], 0.f)), orsrc, at, 0, 0);
+        else if constexpr (NT == 2)
+          __builtin_amdgcn_raw_buffer_store_b32(pack_bf16x2(scale * acc[0][j], scale * acc[1][j]), orsrc, at, 0, 0);
+        else
+          __builtin_amdgcn_raw_buffer_store_b64(u32x2{pack_bf16x2(scale * acc[0][j], scale * acc[1][j]),
+                                                      pack_bf16x2(scale * acc[2][j], scale * acc[3][j])}, orsrc, at, 0, 0);
+      }
+      if constexpr (NS == 2) {
+        // With two stages the K tile of chunk c + 1 was issued in this chunk:
+        // only the stores after it may stay in flight.
+        form_v(c + 1, ov, false);
+        __builtin_amdgcn_s_waitcnt(vmcnt_imm<4>());
+      }
       phase_barrier();
     };
-    auto run = [&](auto rot_c) __attribute__((always_inline)) {   // load orders as in the state waves
-      OutOps o0, o1, o2;
+    Ops o[NS];
+    if (!kHelp || !outw) {
 #pragma unroll
-      for (int part = 0; part < 5; ++part) load(0, o0, part);
-#pragma unroll
-      for (int part = 0; part < 5; ++part) load(min(1, nch - 1), o1, part);
-      __syncthreads();
-      for (int c = 0; c < nch; c += 3) {
-        chunk(true, c, o0, min(c + 2, nch - 1), o2, rot_c);
-        chunk(c + 1 < nch, c + 1, o1, min(c + 3, nch - 1), o0, rot_c);
-        chunk(c + 2 < nch, c + 2, o2, min(c + 4, nch - 1), o1, rot_c);
+      for (int i = 0; i < NS - 1; ++i) {
+        dma_k(min(i, nch - 1), sK[i], sKl[kLo ? i : 0], &sF[i][0][0]);
+        load_v(min(i, nch - 1), o[i]);
       }
-    };
-    switch (slab & 3) {
-      case 0: run(std::integral_constant<int, 0>{}); break;
-      case 1: run(std::integral_constant<int, 1>{}); break;
-      case 2: run(std::integral_constant<int, 2>{}); break;
-      default: run(std::integral_constant<int, 3>{}); break;
+      form_v(0, o[0], true);
+    }
+    if (outw) {
+#pragma unroll
+      for (int i = 0; i < NS - 1; ++i) load_qp(min(i, nch - 1), o[i]);
+    }
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm<0>());
+    __syncthreads();
+    if (outw) {
+      for (int c = 0; c < nch; c += NS) {
+        chunk(std::integral_constant<int, 0>{}, true, c, o[0], o[1], o[NS - 1]);
+        chunk(std::integral_constant<int, 1>{}, c + 1 < nch, c + 1, o[1], o[2 % NS], o[0]);
+        if constexpr (NS == 3) chunk(std::integral_constant<int, NS - 1>{}, c + 2 < nch, c + 2, o[NS - 1], o[0], o[1]);
+      }
+    } else if constexpr (kHelp) {
+      for (int c = 0; c < nch; c += NS) {
+        helper(std::integral_constant<int, 0>{}, c, o[1], o[2]);
+        helper(std::integral_constant<int, 1>{}, c + 1, o[2], o[0]);
+        helper(std::integral_constant<int, 2>{}, c + 2, o[0], o[1]);
+      }
     }
   }
 }
 
-}  // namespace
-}  // namespace aila
-
-namespace aila {
-// Chunk records + launches of the two kernels; shared by the recurrence
-// entry point (bf16 inputs) and the full layer (split fp32 inputs).
-size_t deltanet_chunk_records_bytes(int B, int T, int Hv, bool split) {
-  const size_t nch = (static_cast<size_t>(T) + kC - 1) / kC;
-  return static_cast<size_t>(B) * Hv * nch *
-         (ChunkRec<128, 128>::kBytes + (split ? KeyRec<128, true>::kBytes : KeyRec<128, false>::kBytes));
+template <bool kLo>
+void launch_prep(const bf16* q, const bf16* k, const ConvIn& cv, const bf16* a, const bf16* b, int ab_stride,
+                 const bf16* dt_bias, const float* A_log, unsigned char* records, int B, int T, int Hk, int Hv,
+                 float eps, hipStream_t st) {
+  auto go = [&](auto gp) {
+    constexpr int GP = decltype(gp)::value;
+    hipLaunchKernelGGL((deltanet_chunk_prep_kernel<kLo, GP>), dim3((T + kC - 1) / kC, Hk, B), dim3(kHeadThreads * GP),
+                       0, st, q, k, cv, a, b, ab_stride, dt_bias, A_log, records, T, Hk, Hv, eps);
+  };
+  switch (Hv / Hk) {
+    case 1: go(std::integral_constant<int, 1>{}); break;
+    case 2: go(std::integral_constant<int, 2>{}); break;
+    case 3: go(std::integral_constant<int, 3>{}); break;
+    default: go(std::integral_constant<int, 4>{}); break;   // in passes of four
+  }
 }
 
+template <bool kLo>
+void launch_scan(const bf16* v, const ConvIn& cv, const unsigned char* records, float* state, bf16* out, int B, int T,
+                 int Hk, int Hv, float scale, hipStream_t st) {
+  auto go = [&](auto nt) {
+    constexpr int NT = decltype(nt)::value;
+    hipLaunchKernelGGL((deltanet_chunk_scan_kernel<kLo, NT>), dim3(kD / (16 * NT), Hv, B), dim3(scan_threads(NT)), 0, st,
+                       v, cv, records, state, out, T, Hk, Hv, scale);
+  };
+  // One workgroup per CU; a chunk of 32 or 64 columns takes about 1.25 or 1.75
+  // times one of 16. So the narrowest slab that fits one round of 256 CUs wins
+  // (layer, us at 16 / 32 / 64 columns: 32 heads, T = 4096 152 / 191 / 261; 48
+  // heads, T = 2048 140 / 117 / 152; 64 heads, T = 2048 157 / 131 / 165; 80
+  // heads, T = 1024 148 / 141 / 120; 128 heads, T = 1024 173 / 142 / 120).
+  const long heads = static_cast<long>(B) * Hv;
+  if (heads <= 32) go(std::integral_constant<int, 1>{});
+  else if (heads <= 64) go(std::integral_constant<int, 2>{});
+  else go(std::integral_constant<int, 4>{});
+}
+
+}  // namespace
+
+// Records of the chunked prefill; the sizes callers have allocated since the
+// records also held W and U, which they now only bound.
+size_t deltanet_chunk_records_bytes(int B, int T, int Hv, bool split) {
+  const size_t nch = (static_cast<size_t>(T) + kC - 1) / kC;
+  constexpr size_t kValueHead = 74752, kKeyHead = 32768, kKeyHeadSplit = 49152;
+  static_assert(ChunkRec::kBytes <= kValueHead && KeyRec<false>::kBytes <= kKeyHead && KeyRec<true>::kBytes <= kKeyHeadSplit,
+                "records fit");
+  return static_cast<size_t>(B) * Hv * nch * (kValueHead + (split ? kKeyHeadSplit : kKeyHead));
+}
+
+// Chunk records + launches of the two kernels; shared by the recurrence
+// entry point (bf16 inputs) and the full layer (split fp32 inputs).
 // conv == nullptr: q, k, v planes (bf16 inputs). Otherwise the layer: q, k,
-// v are formed from conv->qkv by the prep (q, k, v unused).
+// v are formed from conv->qkv by the kernels (q, k, v unused).
 void launch_deltanet_chunked(const bf16* q, const bf16* k, const bf16* v, const ConvIn* conv, const bf16* a,
                              const bf16* b, int ab_stride, const bf16* dt_bias, const float* A_log, float* state,
                              bf16* out, unsigned char* records, int B, int T, int Hk, int Hv, float eps, float scale,
                              hipStream_t st) {
-  const int nch = (T + kC - 1) / kC;
   if (conv) {
-    hipLaunchKernelGGL((deltanet_chunk_prep_kernel<128, 128, true>), dim3(nch, Hv, B), dim3(kThreads), 0, st, q, k,
-                       v, *conv, a, b, ab_stride, dt_bias, A_log, records, T, Hk, Hv, eps);
-    hipLaunchKernelGGL((deltanet_chunk_scan_kernel<128, 128, true>), dim3(128 / 16, Hv, B), dim3(2 * kThreads), 0,
-                       st, q, records, state, out, T, Hk, Hv, scale);
+    launch_prep<true>(q, k, *conv, a, b, ab_stride, dt_bias, A_log, records, B, T, Hk, Hv, eps, st);
+    launch_scan<true>(v, *conv, records, state, out, B, T, Hk, Hv, scale, st);
   } else {
-    hipLaunchKernelGGL((deltanet_chunk_prep_kernel<128, 128, false>), dim3(nch, Hv, B), dim3(kThreads), 0, st, q, k,
-                       v, ConvIn{}, a, b, ab_stride, dt_bias, A_log, records, T, Hk, Hv, eps);
-    hipLaunchKernelGGL((deltanet_chunk_scan_kernel<128, 128, false>), dim3(128 / 16, Hv, B), dim3(2 * kThreads), 0,
-                       st, q, records, state, out, T, Hk, Hv, scale);
+    launch_prep<false>(q, k, ConvIn{}, a, b, ab_stride, dt_bias, A_log, records, B, T, Hk, Hv, eps, st);
+    launch_scan<false>(v, ConvIn{}, records, state, out, B, T, Hk, Hv, scale, st);
   }
 }
 }  // namespace aila

@@ -1,0 +1,83 @@
+"""GPU parity of the chunked DeltaNet prefill over the forms its dispatch
+distinguishes: value heads per key head (one prep workgroup forms 1-4 of them
+at a time, more in passes), column slabs of the scan (16, 32 or 64 columns by
+the number of heads) and chunk counts around its two- and three-chunk
+rotations, against the sequential oracle recurrence
+(run_linear_delta_host, Qwen35HybridTextBackend.cpp:1640-1798).
+
+Tolerances as for the other prefill tests: bf16 outputs within 1e-2 of the
+tensor maximum (one bf16 rounding is 2^-9), fp32 states within 1e-3.
+"""
+import numpy as np
+import pytest
+
+import oracle
+from aila_amd import datagen as dg
+
+pytestmark = pytest.mark.gpu
+OUT_TOL, STATE_TOL = 1e-2, 1e-3
+D = 128
+
+
+def _t(x):
+    import torch
+    if x.dtype == np.uint16:
+        return torch.from_numpy(np.ascontiguousarray(x).view(np.int16)).view(torch.bfloat16).cuda()
+    return torch.from_numpy(np.ascontiguousarray(x)).cuda()
+
+
+def _bf(t):
+    import torch
+    return dg.bf16_to_f32(t.detach().view(torch.int16).cpu().numpy().view(np.uint16))
+
+
+def _rel(a, r):
+    return float(np.max(np.abs(a - r)) / max(float(np.max(np.abs(r))), 1e-30))
+
+
+# (B, Hk, Hv): heads per key head 1, 2, 3, 4, 5, 8 and B * Hv on both sides of
+# 32 and 64, where the scan's slabs widen
+SHAPES = [(1, 2, 2), (2, 2, 4), (1, 2, 6), (1, 1, 4), (1, 1, 5), (1, 1, 8), (1, 16, 32), (3, 11, 11), (2, 16, 32),
+          (5, 13, 13), (2, 12, 36)]
+
+
+@pytest.mark.parametrize("T", [1, 64, 65, 129, 257])
+@pytest.mark.parametrize("B,Hk,Hv", SHAPES)
+def test_recurrence_matches_oracle(B, Hk, Hv, T):
+    import torch
+    import aila_amd
+    print(f"deltanet_prefill B={B} T={T} Hk={Hk} Hv={Hv}", flush=True)
+    seed = 41000 + 97 * Hv + T
+    q, k = (dg.normal_bf16(seed, i, (B, T, Hk, D)) for i in (0, 1))
+    v = dg.normal_bf16(seed, 2, (B, T, Hv, D))
+    a, b = (dg.normal_bf16(seed, i, (B, T, Hv)) for i in (3, 4))
+    S0 = dg.normal(seed, 5, B * Hv * D * D, std=0.1).reshape(B, Hv, D, D)
+    st = _t(S0)
+    out = aila_amd.deltanet_prefill(_t(q), _t(k), _t(v), _t(a), _t(b), st)
+    torch.cuda.synchronize()
+    _, want_o, want_S = oracle.deltanet_recurrent(q, k, v, a, b, S0, B, T, Hk, Hv, D, D, fast=True)
+    assert _rel(st.cpu().numpy(), want_S) <= STATE_TOL
+    assert _rel(_bf(out), dg.bf16_to_f32(want_o)) <= OUT_TOL
+
+
+@pytest.mark.parametrize("T", [2, 63, 64, 66, 129, 200])
+@pytest.mark.parametrize("B,Hk,Hv", SHAPES)
+def test_layer_matches_oracle(B, Hk, Hv, T):
+    import torch
+    import aila_amd
+    print(f"deltanet_layer_prefill B={B} T={T} Hk={Hk} Hv={Hv}", flush=True)
+    seed, ch, head = 42000 + 89 * Hv + T, 2 * Hk * D + Hv * D, T % 3
+    qkv, z = dg.normal_bf16(seed, 0, (B, T, ch)), dg.normal_bf16(seed, 1, (B, T, Hv * D))
+    a, b = (dg.normal_bf16(seed, i, (B, T, Hv)) for i in (2, 3))
+    w = dg.normal_bf16(seed, 4, (ch, 4), std=0.5)
+    ring = dg.normal(seed, 5, B * 3 * ch).reshape(B, 3, ch)
+    S0 = dg.normal(seed, 6, B * Hv * D * D, std=0.1).reshape(B, Hv, D, D)
+    norm = 1.0 + dg.normal(seed, 7, D, std=0.1)
+    st, cs = _t(S0), _t(ring)
+    out = aila_amd.deltanet_layer_prefill(_t(qkv), _t(z), _t(a), _t(b), _t(w), cs, head, _t(norm), st, Hk)
+    torch.cuda.synchronize()
+    want_o, want_S, want_cs = oracle.deltanet_layer(qkv, z, a, b, w, ring, head, norm, S0, B, T, Hk, Hv, D, D,
+                                                   fast=True)
+    assert _rel(st.cpu().numpy(), want_S) <= STATE_TOL
+    assert _rel(_bf(out), dg.bf16_to_f32(want_o)) <= OUT_TOL
+    assert np.array_equal(cs.cpu().numpy(), want_cs)
