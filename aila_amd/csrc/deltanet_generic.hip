@@ -1,6 +1,6 @@
 // General-shape Gated DeltaNet: the recurrence and the whole layer for the
 // shapes the tuned kernels do not compile (dk or dv other than their sizes,
-// any conv kernel width, value/key head ratios outside {1, 2, 4}, or a head
+// any conv kernel width, value/key head ratios the tuned kernels do not take (decode: outside 1-4), or a head
 // count that does not divide). Role of the reference's single-workgroup
 // fallback in Qwen35HybridTextBackend::run_linear_delta_decode_gpu
 // (src/models/Qwen35HybridTextBackend.cpp:1168-1304) and of the token loop

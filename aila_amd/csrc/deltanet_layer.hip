@@ -555,8 +555,13 @@ extern "C" int aila_hip_deltanet_layer_decode(const void* qkv, int qkv_stride, c
   AILA_REQUIRE(qkv_stride >= ch && z_stride >= Hv * dv && ab_stride >= Hv,
                "deltanet_layer_decode: row strides too small (qkv %d < %d, z %d, ab %d)", qkv_stride, ch,
                z_stride, ab_stride);
+  // Three value heads to a key head (48 over 16) took the general kernel, which
+  // reads and writes the state in two passes over memory (B = 8, 16 key heads: 31.4 against 9.9 us here);
+  // it still takes such a call whose rows lack the vector alignment.
+  const bool vec = aligned(conv_w, 8) && aligned(z, 8) && z_stride % 4 == 0 && aligned(norm_w, 16) &&
+                   aligned(state, 16) && aligned(out, 8) && aligned(arrivals, 4);
   if (!(dk == kD && dv == kD && conv_kernel == kConvK && Hv % Hk == 0 &&
-        (Hv / Hk == 1 || Hv / Hk == 2 || Hv / Hk == 4))) {
+        (Hv / Hk == 1 || Hv / Hk == 2 || (Hv / Hk == 3 && vec) || Hv / Hk == 4))) {
     // general shapes: one token of the sequential layer kernel, then the
     // ring rewrite
     GenericDeltaNet g{};
@@ -582,8 +587,7 @@ extern "C" int aila_hip_deltanet_layer_decode(const void* qkv, int qkv_stride, c
     g.eps = eps, g.scale = scale;
     return deltanet_generic_launch(g, static_cast<hipStream_t>(stream), "deltanet_layer_decode");
   }
-  AILA_REQUIRE(aligned(conv_w, 8) && aligned(z, 8) && z_stride % 4 == 0 && aligned(norm_w, 16) &&
-                   aligned(state, 16) && aligned(out, 8) && aligned(arrivals, 4),
+  AILA_REQUIRE(vec,
                "deltanet_layer_decode: misaligned conv_w/z/norm_w/state/out/arrivals");
   const int G = Hv / Hk;
   const dim3 grid(Hk, B);
@@ -608,17 +612,19 @@ extern "C" int aila_hip_deltanet_layer_decode(const void* qkv, int qkv_stride, c
   if (arrivals != nullptr && G > 1) {
     switch (G) {
       case 2: AILA_LAYER_DECODE_VH(2); break;
+      case 3: AILA_LAYER_DECODE_VH(3); break;
       case 4: AILA_LAYER_DECODE_VH(4); break;
       default:
-        return set_error(AILA_HIP_EUNSUPPORTED, "deltanet_layer_decode: Hv/Hk = %d not in {1,2,4}", G);
+        return set_error(AILA_HIP_EUNSUPPORTED, "deltanet_layer_decode: Hv/Hk = %d not in {1,2,3,4}", G);
     }
   } else {
     switch (G) {
       case 1: AILA_LAYER_DECODE(1); break;
       case 2: AILA_LAYER_DECODE(2); break;
+      case 3: AILA_LAYER_DECODE(3); break;
       case 4: AILA_LAYER_DECODE(4); break;
       default:
-        return set_error(AILA_HIP_EUNSUPPORTED, "deltanet_layer_decode: Hv/Hk = %d not in {1,2,4}", G);
+        return set_error(AILA_HIP_EUNSUPPORTED, "deltanet_layer_decode: Hv/Hk = %d not in {1,2,3,4}", G);
     }
   }
 #undef AILA_LAYER_DECODE

@@ -323,7 +323,7 @@ int aila_hip_deltanet_decode(const void* q, const void* k, const void* v,
  *   gate: out[b, hv, :] = bf16(rmsnorm(o) * norm_w * silu(z)), rmsnorm over dv,
  *         z row b at z + b*z_stride, norm_w [dv] fp32 (:1153-1160, :153-173).
  * state [B, Hv, dk, dv] fp32 is read and written once. Tuned kernels: dk =
- * dv = 128, conv kernel 4, Hv / Hk in {1, 2, 4} (the reference fast path's
+ * dv = 128, conv kernel 4, Hv / Hk in {1, 2, 3, 4} (the reference fast path's
  * shapes). Other shapes (dk, dv <= 256, conv kernel 1..16, any head counts,
  * key head as aila_hip_deltanet_decode) run the general-shape kernel, the
  * role of the reference's generic fallback (:1168-1304), followed by a

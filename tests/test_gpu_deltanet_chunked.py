@@ -81,3 +81,32 @@ def test_layer_matches_oracle(B, Hk, Hv, T):
     assert _rel(st.cpu().numpy(), want_S) <= STATE_TOL
     assert _rel(_bf(out), dg.bf16_to_f32(want_o)) <= OUT_TOL
     assert np.array_equal(cs.cpu().numpy(), want_cs)
+
+
+@pytest.mark.parametrize("wide", [False, True])
+@pytest.mark.parametrize("B,Hk", [(1, 1), (3, 2), (8, 16)])
+def test_layer_decode_three_value_heads(B, Hk, wide):
+    """Whole-layer decode steps with three value heads to a key head, one
+    workgroup per key head and (arrival counts) one per value head."""
+    import torch
+    import aila_amd
+    Hv, T, head = 3 * Hk, 5, 2
+    seed, ch = 43000 + B, 2 * Hk * D + 3 * Hk * D
+    qkv, z = dg.normal_bf16(seed, 0, (B, T, ch)), dg.normal_bf16(seed, 1, (B, T, Hv * D))
+    a, b = (dg.normal_bf16(seed, i, (B, T, Hv)) for i in (2, 3))
+    w = dg.normal_bf16(seed, 4, (ch, 4), std=0.5)
+    ring = dg.normal(seed, 5, B * 3 * ch).reshape(B, 3, ch)
+    S0 = dg.normal(seed, 6, B * Hv * D * D, std=0.1).reshape(B, Hv, D, D)
+    norm = 1.0 + dg.normal(seed, 7, D, std=0.1)
+    st, cs, wt, nw = _t(S0), _t(ring), _t(w), _t(norm)
+    x = [_t(v) for v in (qkv, z, a, b)]
+    arr = torch.zeros(B * Hk, dtype=torch.int32, device="cuda") if wide else None
+    print(f"deltanet_layer_decode B={B} Hk={Hk} Hv={Hv} wide={wide}", flush=True)
+    outs = [aila_amd.deltanet_layer_decode(*(v[:, t] for v in x), wt, cs, (head + t) % 3, nw, st, Hk, arrivals=arr)
+            for t in range(T)]
+    torch.cuda.synchronize()
+    want_o, want_S, want_cs = oracle.deltanet_layer(qkv, z, a, b, w, ring, head, norm, S0, B, T, Hk, Hv, D, D, fast=True)
+    assert _rel(st.cpu().numpy(), want_S) <= STATE_TOL
+    assert _rel(np.stack([_bf(o) for o in outs], axis=1), dg.bf16_to_f32(want_o)) <= OUT_TOL
+    assert np.array_equal(cs.cpu().numpy(), want_cs)
+    assert arr is None or not arr.any().item()
