@@ -556,7 +556,7 @@ extern "C" int aila_hip_deltanet_layer_decode(const void* qkv, int qkv_stride, c
                "deltanet_layer_decode: row strides too small (qkv %d < %d, z %d, ab %d)", qkv_stride, ch,
                z_stride, ab_stride);
   // Three value heads to a key head (48 over 16) took the general kernel, which
-  // reads and writes the state in two passes over memory (B = 8, 16 key heads: 31.4 against 9.9 us here);
+  // reads and writes the state in two passes over memory (B = 8, 16 key heads: 31.5 against 12.0 us here);
   // it still takes such a call whose rows lack the vector alignment.
   const bool vec = aligned(conv_w, 8) && aligned(z, 8) && z_stride % 4 == 0 && aligned(norm_w, 16) &&
                    aligned(state, 16) && aligned(out, 8) && aligned(arrivals, 4);
@@ -608,14 +608,14 @@ extern "C" int aila_hip_deltanet_layer_decode(const void* qkv, int qkv_stride, c
                      z_stride, ap, bp, ab_stride, wp, conv_state, conv_head, conv_heads, dtp, A_log, norm_w,  \
                      state, op, Hk, eps, scale, arrivals)
   // With an arrivals array and G > 1, one workgroup per value head (more
-  // workgroups in flight); otherwise one per key head.
-  if (arrivals != nullptr && G > 1) {
+  // workgroups in flight); otherwise one per key head. G = 3 ignores the
+  // array, as its callers have been told (general shapes need none).
+  if (arrivals != nullptr && G > 1 && G != 3) {
     switch (G) {
       case 2: AILA_LAYER_DECODE_VH(2); break;
-      case 3: AILA_LAYER_DECODE_VH(3); break;
       case 4: AILA_LAYER_DECODE_VH(4); break;
       default:
-        return set_error(AILA_HIP_EUNSUPPORTED, "deltanet_layer_decode: Hv/Hk = %d not in {1,2,3,4}", G);
+        return set_error(AILA_HIP_EUNSUPPORTED, "deltanet_layer_decode: Hv/Hk = %d not in {2,4}", G);
     }
   } else {
     switch (G) {

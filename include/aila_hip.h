@@ -328,7 +328,7 @@ int aila_hip_deltanet_decode(const void* q, const void* k, const void* v,
  * key head as aila_hip_deltanet_decode) run the general-shape kernel, the
  * role of the reference's generic fallback (:1168-1304), followed by a
  * ring-rewrite launch; conv_state is then [B, K-1, ch] and arrivals is
- * ignored.
+ * ignored, as it is for Hv / Hk = 3.
  *   arrivals  optional device uint32[B*Hk], zero before the first call and
  *             left zero by every call: with it (and Hv > Hk) the layer runs
  *             one workgroup per value head instead of one per key head (the
