@@ -241,7 +241,31 @@ __global__ __launch_bounds__(kThreads) void gqa_decode_split_kernel(
   int t0 = s0 + wave * kChunk;
   int pg_cur = page_of(t0);
   const bool early = PREP && t0 < s1 && t0 + kChunk <= len - 1;
-  if (early) dma_k(0, t0, pg_cur);
+  // So do its V rows: they arrive under the query's norm and rotation (one
+  // sequence at 32768 rows, D = 256: 31.5 -> 30.5 us; the second chunk's K as
+  // well measured no gain).
+  u32x4 vv[kChunk / VR];
+  const int vd = (lane % VL) * 8;
+  const int vr = lane / VL;
+  auto load_v = [&](int t0, int page) __attribute__((always_inline)) {
+    const bf16* Vc = V + row_off(t0, page);
+#pragma unroll
+    for (int i = 0; i < kChunk / VR; ++i) {
+      const int tok = min(t0 + vr + i * VR, s1 - 1) - t0;
+      const bf16* src;
+      if constexpr (WIN) {
+        const int t = t0 + tok;
+        src = V + static_cast<size_t>(t < wsink ? t : t + wgap) * D + vd;
+      } else {
+        src = Vc + static_cast<size_t>(tok) * D + vd;
+      }
+      vv[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src));
+    }
+  };
+  if (early) {
+    dma_k(0, t0, pg_cur);
+    load_v(t0, pg_cur);
+  }
 
   // Query operand (A rows = heads, zero rows for m16 >= G).
   bf16x8_t qa[KS];
@@ -316,8 +340,6 @@ __global__ __launch_bounds__(kThreads) void gqa_decode_split_kernel(
 #pragma unroll
     for (int e = 0; e < 8; ++e) acc[h][e] = 0.f;
   }
-  const int vd = (lane % VL) * 8;
-  const int vr = lane / VL;
 
   // Fused append (decode_prepare's cache write): the workgroup owning the
   // last row writes the new token's K and V there before anything reads it.
@@ -397,20 +419,7 @@ __global__ __launch_bounds__(kThreads) void gqa_decode_split_kernel(
       kb[ks] = *reinterpret_cast<const u32x4*>(ks_base + m16 * (D * 2) + (((ks * 4 + g4) ^ kswz<D>(m16)) << 4));
     // ---- V rows of this chunk: nontemporal register loads, issued before
     //      the next K DMA so waiting on V never waits on that prefetch ------
-    u32x4 vv[kChunk / VR];
-    const bf16* Vc = V + row_off(t0, pg_cur);
-#pragma unroll
-    for (int i = 0; i < kChunk / VR; ++i) {
-      const int tok = min(t0 + vr + i * VR, s1 - 1) - t0;
-      const bf16* src;
-      if constexpr (WIN) {
-        const int t = t0 + tok;
-        src = V + static_cast<size_t>(t < wsink ? t : t + wgap) * D + vd;
-      } else {
-        src = Vc + static_cast<size_t>(tok) * D + vd;
-      }
-      vv[i] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(src));
-    }
+    if (!(PREP && early && it == 0)) load_v(t0, pg_cur);
     const int t_next = t0 + kWaves * kChunk;
     if (t_next < s1) dma_k(stage ^ 1, t_next, pg_nxt);
     // the page of the chunk after next goes out now, used one iteration later
@@ -558,12 +567,16 @@ __global__ __launch_bounds__(kThreads) void gqa_decode_split_kernel(
 // Thread t owns 4 head dims (float4 column c) of the splits i = part (mod P),
 // so its record reads are independent and issued together; the P partial
 // sums meet in LDS.
-template <int D, bool WIN = false>
+// CS workgroups per head, each for D / CS dims: with few heads (a single
+// sequence) one workgroup per head leaves most CUs idle and walks its records in
+// several rounds of loads (16 heads, 128 records each, D = 256: merge 6.0 -> 3.6 us).
+// From 65 heads on one workgroup each fills the chip.
+template <int D, bool WIN = false, int CS = 1>
 __global__ __launch_bounds__(256) void gqa_decode_merge_kernel(
     const float* __restrict__ part, bf16* __restrict__ out, int Hq, int L,
     const int* __restrict__ seq_lens, int len_bias, int split_len, int nsplit, int nsplit_max,
     const bf16* __restrict__ gate, int gate_stride, WinArgs wn) {
-  constexpr int C4 = D / 4;             // float4 columns
+  constexpr int C4 = D / CS / 4;        // float4 columns
   constexpr int P = 256 / C4;           // split phases
   const int hq = blockIdx.x, b = blockIdx.y;
   int len = L;
@@ -576,7 +589,7 @@ __global__ __launch_bounds__(256) void gqa_decode_merge_kernel(
   __shared__ float s_f[kMaxSplits];
   __shared__ float s_inv;
   __shared__ f32x4 s_red[P][C4];
-  const int c = threadIdx.x % C4, ph = threadIdx.x / C4;
+  const int c = threadIdx.x % C4, ph = threadIdx.x / C4, c0 = static_cast<int>(blockIdx.z) * (D / CS);
   constexpr int U = 8;
   // This thread's accumulator rows of the first P*U splits go out before the
   // split factors, so the two rounds of loads overlap.
@@ -584,7 +597,7 @@ __global__ __launch_bounds__(256) void gqa_decode_merge_kernel(
 #pragma unroll
     for (int u = 0; u < U; ++u) {
       const int i = i0 + u * P;
-      v[u] = (i < ns) ? *reinterpret_cast<const f32x4*>(rec0 + static_cast<size_t>(i) * (kRecHeader + D) + kRecHeader + 4 * c)
+      v[u] = (i < ns) ? *reinterpret_cast<const f32x4*>(rec0 + static_cast<size_t>(i) * (kRecHeader + D) + kRecHeader + c0 + 4 * c)
                       : f32x4{0.f, 0.f, 0.f, 0.f};
     }
   };
@@ -642,12 +655,12 @@ __global__ __launch_bounds__(256) void gqa_decode_merge_kernel(
     for (int p2 = 1; p2 < P; ++p2) r += s_red[p2][threadIdx.x];
     r *= s_inv;
     if (gate != nullptr) {   // gated attention: out * sigmoid(gate) (ElementwiseOps.cpp:519-553)
-      const bf16* gr = gate + (static_cast<size_t>(b) * Hq + hq) * gate_stride + 4 * threadIdx.x;
+      const bf16* gr = gate + (static_cast<size_t>(b) * Hq + hq) * gate_stride + c0 + 4 * threadIdx.x;
 #pragma unroll
       for (int j = 0; j < 4; ++j) r[j] *= 1.0f / (1.0f + expf(-bf2f(gr[j])));
     }
     const u32x2 w = {pack_bf16x2(r[0], r[1]), pack_bf16x2(r[2], r[3])};
-    *reinterpret_cast<u32x2*>(out + (static_cast<size_t>(b) * Hq + hq) * D + 4 * threadIdx.x) = w;
+    *reinterpret_cast<u32x2*>(out + (static_cast<size_t>(b) * Hq + hq) * D + c0 + 4 * threadIdx.x) = w;
   }
 }
 
@@ -693,7 +706,12 @@ int launch_decode(const DecodeArgs& a, hipStream_t st) {
                        a.split_len, a.nsplit_max, a.group, scale_log2, a.k_new, a.v_new, a.prep, a.pages, a.win);
   if (a.part) {
     const bool gated = a.prep.q_stride > 0 && a.prep.apply_gate;
-    if (win)
+    constexpr int CS = D / 64;   // 64 dims a workgroup (see the kernel)
+    if (!win && CS > 1 && a.Hq * a.B <= 64)
+      hipLaunchKernelGGL((gqa_decode_merge_kernel<D, false, CS>), dim3(a.Hq, a.B, CS), dim3(256), 0, st, a.part, a.out,
+                         a.Hq, a.L, a.seq_lens, a.len_bias, a.split_len, a.nsplit, a.nsplit_max,
+                         gated ? a.q + D : nullptr, a.prep.q_stride, a.win);
+    else if (win)
       hipLaunchKernelGGL((gqa_decode_merge_kernel<D, true>), dim3(a.Hq, a.B), dim3(256), 0, st, a.part, a.out, a.Hq,
                          a.L, a.seq_lens, a.len_bias, a.split_len, a.nsplit, a.nsplit_max, nullptr, 0, a.win);
     else
