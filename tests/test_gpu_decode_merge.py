@@ -17,8 +17,8 @@ def _t(x):
 
 
 @pytest.mark.parametrize("D", [64, 128, 256])
-@pytest.mark.parametrize("B,Hq,Hkv", [(1, 1, 1), (1, 16, 4), (4, 16, 4), (13, 5, 1), (9, 8, 2)])
-def test_merge_either_side_of_64_heads(B, Hq, Hkv, D):
+@pytest.mark.parametrize("B,Hq,Hkv", [(1, 1, 1), (1, 16, 4), (4, 8, 4), (11, 3, 1), (9, 8, 2)])
+def test_merge_either_side_of_32_heads(B, Hq, Hkv, D):
     import torch
     import aila_amd
     for L in (257, 1100, 4500):
