@@ -26,6 +26,7 @@
 
 #include <algorithm>
 #include <atomic>
+#include <type_traits>
 
 namespace aila {
 namespace {
@@ -563,6 +564,356 @@ __global__ __launch_bounds__(2 * kThreads, 1) void gqa_prefill_kernel(
   }
 }
 
+// o *= f when any != 0 (wave-uniform), with the branch inside the statement: as
+// an `if` around all of O the compiler keeps the rescaled O in registers of its
+// own and copies every one of them before the next products (64 v_mov a phase).
+// The rescale, rare, lies out of line. The s_nops cover the distance that matrix
+// instructions need from O's writers and readers.
+template <int N>
+__device__ __forceinline__ void rescale_if(uint64_t any, f32x4 (&o)[N], float f) {
+  static_assert(N % 2 == 0, "two tiles at a time");
+#pragma unroll
+  for (int i = 0; i < N; i += 2) {
+    float x[8];
+#pragma unroll
+    for (int e = 0; e < 8; ++e) x[e] = o[i + (e >> 2)][e & 3];
+    asm volatile("s_cmp_lg_u64 %9, 0\n\ts_cbranch_scc1 .Lmove%=\n.Lmoved%=:\n\t"
+                 ".subsection 1\n.Lmove%=:\n\ts_nop 15\n\ts_nop 3\n\t"
+                 "v_mul_f32 %0, %0, %8\n\tv_mul_f32 %1, %1, %8\n\tv_mul_f32 %2, %2, %8\n\tv_mul_f32 %3, %3, %8\n\t"
+                 "v_mul_f32 %4, %4, %8\n\tv_mul_f32 %5, %5, %8\n\tv_mul_f32 %6, %6, %8\n\tv_mul_f32 %7, %7, %8\n\t"
+                 "s_nop 7\n\ts_branch .Lmoved%=\n\t.subsection 0"
+                 : "+v"(x[0]), "+v"(x[1]), "+v"(x[2]), "+v"(x[3]), "+v"(x[4]), "+v"(x[5]), "+v"(x[6]), "+v"(x[7])
+                 : "v"(f), "s"(any)
+                 : "scc");
+#pragma unroll
+    for (int e = 0; e < 8; ++e) o[i + (e >> 2)][e & 3] = x[e];
+  }
+}
+
+// D = 256, long prompts and key-split turns: both 4-wave groups of a workgroup
+// share one stream of K/V tiles. The workgroup owns 2 BM consecutive query rows
+// (group A the first BM, B the rest) of a light and a heavy block in turn, every
+// key block serves both groups, and the two keep the ping-pong of the kernel
+// above: B runs one phase behind A, a barrier between phases. Against one stream
+// per group this halves the DMAs a workgroup issues (a vector phase of the kernel
+// above spends 550 of its 1260 cycles issuing eight of them at 64 B/clk) and the
+// K/V bytes it takes from L2, and leaves no partial states to merge; it needs
+// twice the query rows per workgroup.
+// Bound by the LDS: at 16 query rows a wave every MFMA takes its own KiB of
+// operand, 128 KiB a phase at 128 B/clk for 528 cycles of matrix work (16 query
+// heads, S = 8191: 633 -> 587 us, 936 TFLOP/s). D = 128 holds 32 rows a wave, is
+// not bound so, and measured no gain (S = 8192: 503 / 511 us).
+//
+// Four buffers each for K and V. In V(j) group A refills K_{j+3} (its buffer
+// held K_{j-1}, which B read last two phases earlier), group B V_{j+2} (buffer
+// of V_{j-2}); both are waited for in the V phase before their first use, so
+// every DMA has two or more phases to land.
+//
+// The matrix phase streams its operands: V^T of block j-1, then K of block j,
+// each LDS read kPrefetch operands ahead of its MFMA across the boundary.
+template <int D, int RPW, int BN, bool KSPLIT>
+__global__ __launch_bounds__(2 * kThreads, 1) void gqa_prefill_shared_kernel(
+    const bf16* __restrict__ q, int q_row_stride, const bf16* __restrict__ k,
+    const bf16* __restrict__ v, int kv_row_stride, long kv_head_stride,
+    bf16* __restrict__ out, int o_row_stride, int S, int start_pos, int Hkv,
+    int G, float scale_log2, bf16* __restrict__ k_cache,
+    bf16* __restrict__ v_cache, int cache_pos, int max_seq, float* __restrict__ part) {
+  using C = PrefillCfg<D, RPW, BN>;
+  constexpr int BMW = 2 * C::BM;   // query rows of the workgroup
+  constexpr int NB = 4;            // K and V buffers each
+  __shared__ __attribute__((aligned(1024))) unsigned char sK[NB][C::TILE];
+  __shared__ __attribute__((aligned(1024))) unsigned char sV[NB][C::TILE];
+
+  const int grp = __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads);   // 0 = A, 1 = B
+  const int t = threadIdx.x % kThreads, lane = t & 63;
+  const int wave = __builtin_amdgcn_readfirstlane(t >> 6);
+  const int m16 = lane & 15, g4 = lane >> 4;
+
+  // With a key split every workgroup takes one query block and the zs-th of
+  // gridDim.z equal runs of its key blocks; else a light/heavy pair of blocks.
+  const int nqb = (S + BMW - 1) / BMW;
+  const int nx = KSPLIT ? nqb : (nqb + 1) / 2;
+  const int Hq = static_cast<int>(gridDim.y), nz = KSPLIT ? static_cast<int>(gridDim.z) : 1;
+  const int nwg = nx * Hq * nz;
+  const int lin = blockIdx.x + nx * (blockIdx.y + Hq * blockIdx.z);
+  int logical = lin;   // XCD-aware order, as in the kernel above
+  if (nwg % kNumXcd == 0) logical = (lin % kNumXcd) * (nwg / kNumXcd) + lin / kNumXcd;
+  const int pr = logical % nx;
+  const int h = (logical / nx) % Hq;
+  const int zs = KSPLIT ? logical / (nx * Hq) : 0;
+  const int kvh = h / G;
+  const int ql = pr, qh = KSPLIT ? pr : nqb - 1 - pr;    // light / heavy query block
+  auto nkeyblk = [&](int qb) __attribute__((always_inline)) { return (start_pos + min((qb + 1) * BMW, S) - 1) / BN + 1; };
+  const int nl = (ql < qh) ? nkeyblk(ql) : 0;            // a middle block pairs with itself
+  const int h0 = KSPLIT ? nkeyblk(qh) * zs / nz : 0;
+  const int nh = (KSPLIT ? nkeyblk(qh) * (zs + 1) / nz : nkeyblk(qh)) - h0;
+  const int N = nl + nh;
+  auto kb_of = [&](int it) __attribute__((always_inline)) { return it < nl ? it : h0 + it - nl; };
+  const int kv_len = start_pos + S;
+  const bf16* Kh = k + static_cast<size_t>(kvh) * kv_head_stride;
+  const bf16* Vh = v + static_cast<size_t>(kvh) * kv_head_stride;
+
+  // K/V block -> LDS by DMA, by the four waves of one group (see above)
+  static_assert(C::LOADS <= 8, "dma_off extent");
+  int off[8];
+#pragma unroll
+  for (int i = 0; i < C::LOADS; ++i) {
+    const int p = (i * kWaves + wave) * 64 + lane;
+    const int r = p / C::NC;
+    off[i] = (r * kv_row_stride + ((p % C::NC) ^ (grp == 0 ? swz_k<D>(r) : swz_v<D>(r))) * 8) * 2;
+  }
+  // group A issues K tiles, group B V tiles
+  auto issue_tile = [&](unsigned char* tile, int kb) __attribute__((always_inline)) {
+    const int key0 = kb * BN;
+    const u32x4 src = buffer_rsrc((grp == 0 ? Kh : Vh) + static_cast<size_t>(key0) * kv_row_stride,
+                                  min(kv_len - key0, BN) * kv_row_stride * 2);
+#pragma unroll
+    for (int i = 0; i < C::LOADS; ++i) dma16_to_lds(src, off[i], tile + (i * kWaves + wave) * 64 * 16);
+  };
+
+  bf16x8_t qb_op[C::QT][C::KS];
+  f32x4 o_acc[C::QT][C::DT];
+  float m_run[C::QT], l_run[C::QT];
+  int row0 = 0;                    // first query row of this wave's current segment
+  auto begin_segment = [&](int qb) __attribute__((always_inline)) {
+    row0 = qb * BMW + grp * C::BM + wave * RPW;
+#pragma unroll
+    for (int qt = 0; qt < C::QT; ++qt) {
+      const int row = min(row0 + qt * 16 + m16, S - 1);
+      const bf16* qr = q + static_cast<size_t>(row) * q_row_stride + h * D + g4 * 8;
+#pragma unroll
+      for (int ks = 0; ks < C::KS; ++ks) qb_op[qt][ks] = as_bf16x8(ld16(qr + ks * 32));
+      m_run[qt] = -INFINITY;
+      l_run[qt] = 0.f;
+#pragma unroll
+      for (int dt = 0; dt < C::DT; ++dt) o_acc[qt][dt] = f32x4{0.f, 0.f, 0.f, 0.f};
+    }
+  };
+  auto store_segment = [&]() __attribute__((always_inline)) {
+#pragma unroll
+    for (int qt = 0; qt < C::QT; ++qt) {
+      const int row = row0 + qt * 16 + m16;
+      if (row < S) {
+        if constexpr (KSPLIT) {   // the unnormalised state, as in the kernel above
+          float* rec = part + ((static_cast<size_t>(zs) * Hq + h) * S + row) * (D + 4);
+          if (g4 == 0) *reinterpret_cast<f32x4*>(rec) = f32x4{m_run[qt], l_run[qt], 0.f, 0.f};
+#pragma unroll
+          for (int dt = 0; dt < C::DT; ++dt)
+            *reinterpret_cast<f32x4*>(rec + 4 + dt * 16 + g4 * 4) = o_acc[qt][dt];
+        } else {
+          const float inv = 1.0f / l_run[qt];   // full row sum, held by every lane
+          bf16* orow = out + static_cast<size_t>(row) * o_row_stride + h * D + g4 * 4;
+#pragma unroll
+          for (int dt = 0; dt < C::DT; ++dt) {
+            const f32x4 o = o_acc[qt][dt] * inv;
+            const u32x2 w = {pack_bf16x2(o[0], o[1]), pack_bf16x2(o[2], o[3])};
+            __builtin_nontemporal_store(w, reinterpret_cast<u32x2*>(orow + dt * 16));
+          }
+        }
+      }
+    }
+  };
+
+  // ---- matrix phase ---------------------------------------------------------
+  constexpr int NV = C::PS * C::DT, NK = C::KS * C::KT;
+  // S^T accumulators: at least four independent chains
+  constexpr int CH = C::KT * C::QT < 4 ? 2 : 1;
+  f32x4 st[C::KT][C::QT];
+  bf16x8_t pb[C::PS][C::QT];   // step s2 covers keys 32*s2 + {4g..4g+3, 16+4g..16+4g+3}
+  int s_key0 = 0;
+  auto matrix = [&](auto pv_c, auto s_c, const unsigned char* tv, const unsigned char* tk) __attribute__((always_inline)) {
+    constexpr bool PV = decltype(pv_c)::value, SB = decltype(s_c)::value;
+    constexpr int n0 = PV ? NV : 0, n = n0 + (SB ? NK : 0);
+    const int vr = 4 * g4 + (m16 >> 2);          // V row within a 32-key step (first half)
+    const int vc = 4 * (m16 & 3);                // column offset within a 16-wide d tile
+    auto load_op = [&](int i) __attribute__((always_inline)) {
+      if (i < n0) {                              // V^T operand (s2, dt) by transposing reads
+        const int s2 = i / C::DT, dt = i % C::DT;
+        const int d = dt * 16 + vc;
+        const int r0 = s2 * 32 + vr, r1 = r0 + 16;
+        const u32x2 lo = ds_read_tr4(tv + r0 * C::RB + (((d >> 3) ^ swz_v<D>(r0)) << 4) + ((d & 7) << 1));
+        const u32x2 hi = ds_read_tr4(tv + r1 * C::RB + (((d >> 3) ^ swz_v<D>(r1)) << 4) + ((d & 7) << 1));
+        return as_bf16x8(u32x4{lo[0], lo[1], hi[0], hi[1]});
+      }
+      const int ks = (i - n0) / C::KT, kt = (i - n0) % C::KT;   // K operand
+      const int r = kt * 16 + m16;
+      return as_bf16x8(*reinterpret_cast<const u32x4*>(tk + r * C::RB + (((ks * 4 + g4) ^ swz_k<D>(r)) << 4)));
+    };
+    bf16x8_t op[n];
+#pragma unroll
+    for (int i = 0; i < kPrefetch && i < n; ++i) op[i] = load_op(i);
+    if constexpr (PV) {
+      // row sums of P while the first reads are in flight: a ones A operand
+      // gives every lane the full row sum of its query
+      const bf16x8_t ones = as_bf16x8(u32x4{0x3F803F80u, 0x3F803F80u, 0x3F803F80u, 0x3F803F80u});
+#pragma unroll
+      for (int qt = 0; qt < C::QT; ++qt) {
+        f32x4 ls = {0.f, 0.f, 0.f, 0.f};
+#pragma unroll
+        for (int s2 = 0; s2 < C::PS; ++s2) ls = mfma16x16x32(ones, pb[s2][qt], ls);
+        l_run[qt] += ls[0];
+      }
+    }
+    f32x4 sc[C::KT][C::QT][CH];
+#pragma unroll
+    for (int kt = 0; kt < C::KT; ++kt)
+#pragma unroll
+      for (int qt = 0; qt < C::QT; ++qt)
+#pragma unroll
+        for (int ch = 0; ch < CH; ++ch) sc[kt][qt][ch] = f32x4{0.f, 0.f, 0.f, 0.f};
+    __builtin_amdgcn_sched_barrier(0);
+#pragma unroll
+    for (int i = 0; i < n; ++i) {
+      if (i + kPrefetch < n) op[i + kPrefetch] = load_op(i + kPrefetch);
+      if (i < n0) {
+        const int s2 = i / C::DT, dt = i % C::DT;
+#pragma unroll
+        for (int qt = 0; qt < C::QT; ++qt) o_acc[qt][dt] = mfma16x16x32(op[i], pb[s2][qt], o_acc[qt][dt]);
+      } else {
+        const int ks = (i - n0) / C::KT, kt = (i - n0) % C::KT;
+#pragma unroll
+        for (int qt = 0; qt < C::QT; ++qt)
+          sc[kt][qt][ks % CH] = mfma16x16x32(op[i], qb_op[qt][ks], sc[kt][qt][ks % CH]);
+      }
+      __builtin_amdgcn_sched_barrier(0);
+    }
+    if constexpr (SB) {
+#pragma unroll
+      for (int kt = 0; kt < C::KT; ++kt)
+#pragma unroll
+        for (int qt = 0; qt < C::QT; ++qt) {
+          st[kt][qt] = sc[kt][qt][0];
+          if constexpr (CH == 2) st[kt][qt] += sc[kt][qt][1];
+        }
+    }
+  };
+
+  // ---- vector phase: softmax of S_j into P_j (as in the kernel above) ---------
+  auto softmax = [&](const bool masked) __attribute__((always_inline)) {
+    if (masked) {
+#pragma unroll
+      for (int qt = 0; qt < C::QT; ++qt) {
+        const int rel = start_pos + row0 + qt * 16 + m16 - s_key0 - g4 * 4;   // key offset limit
+#pragma unroll
+        for (int kt = 0; kt < C::KT; ++kt)
+#pragma unroll
+          for (int j = 0; j < 4; ++j)
+            if (kt * 16 + j > rel) st[kt][qt][j] = -INFINITY;
+      }
+    }
+    auto exp_pass = [&]() __attribute__((always_inline)) {
+#pragma unroll
+      for (int qt = 0; qt < C::QT; ++qt) {
+        const float nm = (m_run[qt] == -INFINITY) ? 0.f : -m_run[qt];
+#pragma unroll
+        for (int s2 = 0; s2 < C::PS; ++s2) {
+          float p[8];
+#pragma unroll
+          for (int j = 0; j < 4; ++j) {
+            p[j] = fast_exp2(fmaf(st[2 * s2][qt][j], scale_log2, nm));
+            p[4 + j] = fast_exp2(fmaf(st[2 * s2 + 1][qt][j], scale_log2, nm));
+          }
+          pb[s2][qt] = as_bf16x8(u32x4{pack_bf16x2(p[0], p[1]), pack_bf16x2(p[2], p[3]),
+                                       pack_bf16x2(p[4], p[5]), pack_bf16x2(p[6], p[7])});
+        }
+      }
+    };
+    exp_pass();
+    float alpha[C::QT];
+    bool any_rescale = false;
+#pragma unroll
+    for (int qt = 0; qt < C::QT; ++qt) {
+      float mx = -INFINITY;
+#pragma unroll
+      for (int kt = 0; kt < C::KT; ++kt)
+#pragma unroll
+        for (int j = 0; j < 4; ++j) mx = fmaxf(mx, st[kt][qt][j]);
+      mx = xrow4_max(mx) * scale_log2;
+      const bool grow = mx > m_run[qt] + kLazyRescaleLog2;
+      const float mn = grow ? mx : m_run[qt];
+      alpha[qt] = grow ? ((m_run[qt] == -INFINITY) ? 0.f : fast_exp2(m_run[qt] - mn)) : 1.0f;
+      m_run[qt] = mn;
+      any_rescale |= grow;
+    }
+    // o_acc and l hold every block before j (M(j) added P_{j-1}).
+    const uint64_t any = __builtin_amdgcn_ballot_w64(any_rescale);
+    if (any != 0) {
+      exp_pass();
+#pragma unroll
+      for (int qt = 0; qt < C::QT; ++qt) l_run[qt] *= alpha[qt];
+    }
+#pragma unroll
+    for (int qt = 0; qt < C::QT; ++qt) rescale_if(any, o_acc[qt], alpha[qt]);
+  };
+
+  // ---- prologue: K_0..K_2 (A), V_0, V_1 (B) -----------------------------------
+  const int ahead = grp == 0 ? 3 : 2;
+  unsigned char* const mine = grp == 0 ? sK[0] : sV[0];   // the ring this group fills
+#pragma unroll
+  for (int i = 0; i < 3; ++i)
+    if (i < ahead && i < N) issue_tile(mine + i * C::TILE, kb_of(i));
+  __builtin_amdgcn_s_waitcnt(vmcnt_imm<0>());
+  __syncthreads();
+
+  constexpr std::integral_constant<bool, true> yes{};
+  constexpr std::integral_constant<bool, false> no{};
+  auto ktile = [&](int j) __attribute__((always_inline)) { return sK[0] + (j & (NB - 1)) * C::TILE; };
+  auto vtile = [&](int j) __attribute__((always_inline)) { return sV[0] + (j & (NB - 1)) * C::TILE; };
+  // V(j) between its two barriers. Blocks wholly in a wave's future are masked
+  // like the diagonal one (their P is zero).
+  auto vector = [&](int j) __attribute__((always_inline)) {
+    phase_barrier();
+    const int jn = j + ahead;
+    if (jn < N) issue_tile(mine + (jn & (NB - 1)) * C::TILE, kb_of(jn));
+    s_key0 = kb_of(j) * BN;
+    softmax(s_key0 + BN - 1 > start_pos + row0);
+    // K_{j+1} (A, two tiles issued since) or V_{j+1} (B, one) must have landed
+    if (grp == 0 && jn < N) __builtin_amdgcn_s_waitcnt(vmcnt_imm<2 * C::LOADS>());
+    else if (grp == 0 ? jn - 1 < N : jn < N) __builtin_amdgcn_s_waitcnt(vmcnt_imm<C::LOADS>());
+    else __builtin_amdgcn_s_waitcnt(vmcnt_imm<0>());
+    phase_barrier();
+  };
+  if (grp == 1) phase_barrier();   // group B runs one phase behind
+  int j = 0;
+#pragma unroll 1
+  for (int seg = nl > 0 ? 0 : 1; seg < 2; ++seg) {   // light block, heavy block
+    const int end = seg == 0 ? nl : N;
+    begin_segment(seg == 0 ? ql : qh);
+    if (j < end) {
+      matrix(no, yes, vtile(j), ktile(j));
+      vector(j);
+#pragma unroll 1
+      for (++j; j < end; ++j) {
+        matrix(yes, yes, vtile(j - 1), ktile(j));
+        vector(j);
+      }
+      matrix(yes, no, vtile(j - 1), ktile(j));
+    }
+    store_segment();   // the next segment's first S follows in the same phase
+  }
+  phase_barrier();
+  // fused copy_to_cache: the K/V rows of this workgroup's query blocks, shared
+  // by the G query heads of the KV group (head h copies every G-th row)
+  if (!KSPLIT && k_cache != nullptr) {
+    const int gi = h % G;
+#pragma unroll 1
+    for (int pass = 0; pass < 2; ++pass) {
+      const int qb = pass == 0 ? qh : ql;
+      if (pass == 1 && ql == qh) break;
+      const int r0 = qb * BMW, r1 = min(r0 + BMW, S);
+      const int nrow = (r1 - r0 - gi + G - 1) / G;   // rows r0 + gi, r0 + gi + G, ...
+      for (int p = threadIdx.x; p < nrow * C::NC; p += 2 * kThreads) {
+        const int row = r0 + gi + (p / C::NC) * G, c = p % C::NC;
+        const size_t src = static_cast<size_t>(row) * kv_row_stride + c * 8;
+        const size_t dst = (static_cast<size_t>(kvh) * max_seq + cache_pos + row) * D + c * 8;
+        __builtin_nontemporal_store(ld16(Kh + src), reinterpret_cast<u32x4*>(k_cache + dst));
+        __builtin_nontemporal_store(ld16(Vh + src), reinterpret_cast<u32x4*>(v_cache + dst));
+      }
+    }
+  }
+  if (grp == 0) phase_barrier();   // group B's last phase
+}
+
 // Key-split merge: out row = sum_z 2^(m_z - M) acc_z / sum_z 2^(m_z - M) l_z
 // over the slices' partial records (M = max m_z; a slice whose keys were
 // all masked for the row has m = -inf and weight 0). D/4 threads per
@@ -598,6 +949,30 @@ __global__ __launch_bounds__(256) void gqa_prefill_merge_kernel(const float* __r
       u32x2{pack_bf16x2(acc[0] * inv, acc[1] * inv), pack_bf16x2(acc[2] * inv, acc[3] * inv)};
 }
 
+template <int D>
+int prefill_resident();
+
+// D = 256: whether the kernel whose groups share their K/V tiles takes an unsplit
+// prefill. Its step (128 query rows by 32 keys) takes about 0.93 of the other
+// kernel's (two groups of 64 rows by 32 keys), but its workgroups are half as
+// many and twice as long, so it loses where they leave a round of the device
+// partly empty. Measured, us, other kernel / this one, 16 query heads: S = 2048
+// (128 workgroups) 60 / 87, 3072 (192) 128 / 134, 3500 (224) 148 / 137, 4096
+// (256) 171 / 162, 4400 (288) 262 / 319, 6000 (384) 356 / 418, 7000 (448) 535 /
+// 481, 8191 (512) 633 / 587, 12000 (752) 1364 / 1267; 32 heads, S = 2048 97 / 96.
+bool shared_tiles(int S, int start_pos, int Hq) {
+  const long cus = prefill_resident<256>();   // one workgroup of either kernel a CU
+  const long n64 = (S + 63) / 64, n128 = (S + 127) / 128, prefix = start_pos / 32;
+  const long wg = (n128 + 1) / 2 * Hq, rounds = (wg + cus - 1) / cus;
+  const long steps = rounds * (4 * (n128 + 1) + 2 * prefix);
+  const long other = ((n64 + 1) / 2 * Hq + cus - 1) / cus * (n64 + 1 + prefix);
+  return wg * 100 >= 85 * rounds * cus && steps * 95 < other * 100;
+}
+// ... and a key-split one, where both kernels launch the same workgroups as long
+// as 128-row blocks pad no more than 64-row ones do (S = 250 over 7900 rows 66 ->
+// 57 us, 512 over 4096 62 -> 57; 300 over 16000, five 64-row blocks, 165 / 192).
+bool shared_split(int S) { return (S + 63) / 64 % 2 == 0; }
+
 template <int D, int RPW, int BN>
 int launch_prefill(const bf16* q, const bf16* k, const bf16* v, int kv_row_stride,
                    long kv_head_stride, bf16* out, int S, int start_pos, int Hq,
@@ -616,14 +991,20 @@ int launch_prefill(const bf16* q, const bf16* k, const bf16* v, int kv_row_strid
     nz = 1;
     part = nullptr;
   }
-  if (part == nullptr)
-    hipLaunchKernelGGL((gqa_prefill_kernel<D, RPW, BN, false>), dim3(npair, Hq), dim3(2 * kThreads), 0, st,
-                       q, Hq * D, k, v, kv_row_stride, kv_head_stride, out, Hq * D, S, start_pos,
-                       Hkv, Hq / Hkv, scale_log2, k_cache, v_cache, cache_pos, max_seq, nullptr);
-  else
-    hipLaunchKernelGGL((gqa_prefill_kernel<D, RPW, BN, true>), dim3(npair, Hq, nz), dim3(2 * kThreads), 0, st,
-                       q, Hq * D, k, v, kv_row_stride, kv_head_stride, out, Hq * D, S, start_pos,
-                       Hkv, Hq / Hkv, scale_log2, nullptr, nullptr, 0, max_seq, part);
+  const auto go = [&](auto kernel, dim3 grid) {
+    const bool split = part != nullptr;   // a split call writes records, no cache rows
+    hipLaunchKernelGGL(kernel, grid, dim3(2 * kThreads), 0, st, q, Hq * D, k, v, kv_row_stride, kv_head_stride, out,
+                       Hq * D, S, start_pos, Hkv, Hq / Hkv, scale_log2, split ? nullptr : k_cache,
+                       split ? nullptr : v_cache, split ? 0 : cache_pos, max_seq, part);
+  };
+  const bool shared = D == 256 && (part != nullptr ? shared_split(S) : shared_tiles(S, start_pos, Hq));
+  if constexpr (D == 256) {
+    const int nb = (S + 2 * C::BM - 1) / (2 * C::BM);
+    if (shared && part == nullptr) go(gqa_prefill_shared_kernel<D, RPW, BN, false>, dim3((nb + 1) / 2, Hq));
+    else if (shared) go(gqa_prefill_shared_kernel<D, RPW, BN, true>, dim3(nb, Hq, nz));
+  }
+  if (!shared && part == nullptr) go(gqa_prefill_kernel<D, RPW, BN, false>, dim3(npair, Hq));
+  else if (!shared) go(gqa_prefill_kernel<D, RPW, BN, true>, dim3(npair, Hq, nz));
   if (part != nullptr) {
     constexpr int RPB = 256 / (D / 4);
     const long rows = static_cast<long>(S) * Hq;
