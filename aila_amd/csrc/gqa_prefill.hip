@@ -599,10 +599,10 @@ __device__ __forceinline__ void rescale_if(uint64_t any, f32x4 (&o)[N], float f)
 // above spends 550 of its 1260 cycles issuing eight of them at 64 B/clk) and the
 // K/V bytes it takes from L2, and leaves no partial states to merge; it needs
 // twice the query rows per workgroup.
-// Bound by the LDS: at 16 query rows a wave every MFMA takes its own KiB of
-// operand, 128 KiB a phase at 128 B/clk for 528 cycles of matrix work (16 query
-// heads, S = 8191: 633 -> 587 us, 936 TFLOP/s). D = 128 holds 32 rows a wave, is
-// not bound so, and measured no gain (S = 8192: 503 / 511 us).
+// Bound by the operand reads: at 16 query rows a wave every MFMA takes its own
+// KiB from the LDS, 128 KiB in a matrix phase of 1430 cycles with 528 of MFMA (16
+// query heads, S = 8191: 633 -> 587 us, 936 TFLOP/s). D = 128 holds 32 rows a
+// wave and measured no gain (S = 8192: 503 / 511 us).
 //
 // Four buffers each for K and V. In V(j) group A refills K_{j+3} (its buffer
 // held K_{j-1}, which B read last two phases earlier), group B V_{j+2} (buffer
