@@ -128,11 +128,12 @@ __global__ __launch_bounds__(kThreads) void gqa_decode_split_kernel(
   static_assert(D % 32 == 0 && D <= 256, "D");
   static_assert(!(PAGED && PREP), "the paged variant has no fused preparation");
   static_assert(!(WIN && (PAGED || PREP)), "the window variant is contiguous and has no fused append");
-  static_assert(G == 1 || G == 2 || G == 4 || G == 8, "G");
+  static_assert(G >= 1 && G <= 8, "G");
   constexpr int KS = D / 32;          // MFMA k-steps over the head dim
   constexpr int VL = D / 8;           // lanes per V row (16 B each)
   constexpr int VR = 64 / VL;         // V rows per load instruction
   constexpr int GR = (G + 3) / 4;     // 16-lane rows holding score heads
+  constexpr int GP = G <= 2 ? G : GR * 4;   // heads per row of the P slice (whole 16-byte reads)
   constexpr int NC = D / 8;           // 16-byte chunks per row
   constexpr int STAGE = kChunk * D * 2;          // bytes of one K stage (16 rows)
   constexpr int NDMA = STAGE / 1024;             // DMA instructions per stage per wave
@@ -207,7 +208,7 @@ __global__ __launch_bounds__(kThreads) void gqa_decode_split_kernel(
   };
 
   __shared__ __attribute__((aligned(1024))) unsigned char s_k[kWaves][2][STAGE];
-  __shared__ float s_p[kWaves][kChunk][G];
+  __shared__ __attribute__((aligned(16))) float s_p[kWaves][kChunk][GP];
   __shared__ float s_ml[kWaves][2][G];
   __shared__ float s_q[PREP ? G : 1][PREP ? D : 1];   // prepared q (fused preparation only)
   __shared__ float s_tab[PREP ? D : 1];               // (cos, sin) per rotary pair
@@ -677,7 +678,7 @@ struct DecodeArgs {
   const int* seq_lens;
   int len_bias;          // sequence b attends min(seq_lens[b] + len_bias, L) rows
   int split_len, nsplit, nsplit_max;
-  int group, chunks;     // Hq / Hkv, and workgroups per KV head (group / tile, rounded up)
+  int group, tile, chunks;   // Hq / Hkv, query heads per workgroup, workgroups per KV head (group / tile, rounded up)
   const bf16* k_new;     // fused append (null: none)
   const bf16* v_new;
   PrepArgs prep;         // q_stride = 0: no fused preparation
@@ -689,23 +690,17 @@ template <int D, int G>
 int launch_decode(const DecodeArgs& a, hipStream_t st) {
   const float scale_log2 = kLog2e / sqrtf(static_cast<float>(D));
   const bool win = a.win.window > 0;
-  if (a.prep.q_stride > 0)
-    hipLaunchKernelGGL((gqa_decode_split_kernel<D, G, true>), dim3(a.nsplit, a.Hkv * a.chunks, a.B), dim3(kThreads), 0, st,
-                       a.q, a.kc, a.vc, a.out, a.part, a.Hq, a.Hkv, a.max_seq, a.L, a.seq_lens, a.len_bias,
-                       a.split_len, a.nsplit_max, a.group, scale_log2, a.k_new, a.v_new, a.prep, a.pages, a.win);
-  else if (a.pages.table != nullptr)
-    hipLaunchKernelGGL((gqa_decode_split_kernel<D, G, false, true>), dim3(a.nsplit, a.Hkv * a.chunks, a.B), dim3(kThreads), 0,
-                       st, a.q, a.kc, a.vc, a.out, a.part, a.Hq, a.Hkv, a.max_seq, a.L, a.seq_lens, a.len_bias,
-                       a.split_len, a.nsplit_max, a.group, scale_log2, a.k_new, a.v_new, a.prep, a.pages, a.win);
-  else if (win)
-    hipLaunchKernelGGL((gqa_decode_split_kernel<D, G, false, false, true>), dim3(a.nsplit, a.Hkv * a.chunks, a.B),
-                       dim3(kThreads), 0, st, a.q, a.kc, a.vc, a.out, a.part, a.Hq, a.Hkv, a.max_seq, a.L,
-                       a.seq_lens, a.len_bias, a.split_len, a.nsplit_max, a.group, scale_log2, a.k_new, a.v_new, a.prep,
-                       a.pages, a.win);
-  else
-    hipLaunchKernelGGL((gqa_decode_split_kernel<D, G>), dim3(a.nsplit, a.Hkv * a.chunks, a.B), dim3(kThreads), 0, st,
-                       a.q, a.kc, a.vc, a.out, a.part, a.Hq, a.Hkv, a.max_seq, a.L, a.seq_lens, a.len_bias,
-                       a.split_len, a.nsplit_max, a.group, scale_log2, a.k_new, a.v_new, a.prep, a.pages, a.win);
+  auto go = [&](auto kernel) {
+    hipLaunchKernelGGL(kernel, dim3(a.nsplit, a.Hkv * a.chunks, a.B), dim3(kThreads), 0, st, a.q, a.kc, a.vc, a.out,
+                       a.part, a.Hq, a.Hkv, a.max_seq, a.L, a.seq_lens, a.len_bias, a.split_len, a.nsplit_max, a.group,
+                       scale_log2, a.k_new, a.v_new, a.prep, a.pages, a.win);
+  };
+  if (a.pages.table != nullptr) go(gqa_decode_split_kernel<D, G, false, true>);
+  else if constexpr (D != 128 || G != 7) {   // see decode_tile
+    if (a.prep.q_stride > 0) go(gqa_decode_split_kernel<D, G, true>);
+    else if (win) go(gqa_decode_split_kernel<D, G, false, false, true>);
+    else go(gqa_decode_split_kernel<D, G>);
+  }
   if (a.part) {
     const bool gated = a.prep.q_stride > 0 && a.prep.apply_gate;
     constexpr int CS = D / 64;   // 64 dims a workgroup (see the kernel)
@@ -724,10 +719,20 @@ int launch_decode(const DecodeArgs& a, hipStream_t st) {
   return check_launch("gqa_decode");
 }
 
-// Query-head tile of the split kernel for a group of g query heads per KV
-// head: the smallest of 1, 2, 4, 8 that holds it, else 8 (several
-// workgroups per KV head, each streaming its K/V; see the kernel).
-int decode_tile(int g) { return g <= 1 ? 1 : g <= 2 ? 2 : g <= 4 ? 4 : 8; }
+// Query-head tile of the split kernel for a group of g query heads per KV head:
+// ceil(g / 8) workgroups per KV head, each streaming its K/V, share the group
+// evenly. A tile's P.V and its accumulators cost VALU time and registers whether
+// its rows are used or not (tile 8 at D = 256 leaves one workgroup a CU, tile 6
+// two), so each has its own size (us, rounded up to 1, 2, 4, 8 -> own; B = 8, 4 KV
+// heads, 4096 rows at D = 256: ratio 3 29.0 -> 28.3, 5 34.6 -> 30.7, 6 34.7 ->
+// 31.8, 9 56.5 -> 37.6, 12 57.0 -> 39.3; 8192 rows, D = 64: 5 25.0 -> 20.7, 12 35.9
+// -> 33.5; D = 128: 3 28.8 -> 27.9, 5 31.5 -> 30.5, 12 44.9 -> 39.4, paged ratio 5
+// 35.0 -> 29.6). Only at D = 128 over a contiguous cache is 7 no faster than in a
+// tile of 8 (32.9 / 32.2; paged 32.8 / 35.4).
+int decode_tile(int g, int D, bool paged) {
+  const int chunks = (g + 7) / 8, tile = (g + chunks - 1) / chunks;
+  return tile == 7 && D == 128 && !paged ? 8 : tile;
+}
 
 // Workgroups of the split kernel that the device holds at once (occupancy x
 // CUs), per device, computed on first use. The split count targets exactly
@@ -737,30 +742,43 @@ int decode_tile(int g) { return g <= 1 ? 1 : g <= 2 ? 2 : g <= 4 ? 4 : 8; }
 // The per-device value is idempotent, so concurrent first calls may both
 // compute it; the atomic makes the publication race-free.
 template <int D, int G>
-int resident_workgroups() {
+int resident_workgroups(int max_per_cu) {
   constexpr int kMaxDev = 64;
-  static std::atomic<int> cache[kMaxDev];
+  static std::atomic<int> cache[kMaxDev];   // workgroups per CU << 16 | CUs
   int dev = 0;
   if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) return 512;
-  const int known = cache[dev].load(std::memory_order_relaxed);
-  if (known > 0) return known;
-  int per_cu = 0, cus = 0;
-  if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gqa_decode_split_kernel<D, G>, kThreads, 0) != hipSuccess ||
-      hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || per_cu <= 0 || cus <= 0)
-    return 512;
-  cache[dev].store(per_cu * cus, std::memory_order_relaxed);
-  return per_cu * cus;
+  int known = cache[dev].load(std::memory_order_relaxed);
+  if (known <= 0) {
+    int per_cu = 0, cus = 0;
+    if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gqa_decode_split_kernel<D, G>, kThreads, 0) !=
+            hipSuccess ||
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || per_cu <= 0 || cus <= 0)
+      return 512;
+    known = per_cu << 16 | cus;
+    cache[dev].store(known, std::memory_order_relaxed);
+  }
+  return std::min(known >> 16, max_per_cu) * (known & 0xffff);
 }
 
-int resident_for(int D, int G) {
+// The plan's workgroups for one round. Three a CU stream no faster than two at
+// D = 128 (tiles 3 and 4: B = 8, 4 KV heads, 16384 rows 5% slower; tile 6 over two
+// workgroups a KV head 54 / 39 us), and the paged kernel, with up to 10 registers
+// more, would not hold them all at once (tile 2, 16384 rows: 12% slower; tile 6:
+// 40 / 31 us); tile 1 and 2 over a contiguous cache measured within 3% either way.
+// At D = 64 tiles 3 and 5 to 7 take three, as tile 8 does (paged tile 3 at 16384
+// rows 13% slower otherwise); 1, 2 and 4 measured up to 10% faster with all theirs.
+int resident_for(int D, int tile, bool paged) {
+  const int cap = D == 64 ? (tile == 3 || tile > 4 ? 3 : 8) : D == 128 && (paged || tile >= 3) ? 2 : 8;
   auto pick = [&](auto d_tag) -> int {
     constexpr int DD = decltype(d_tag)::value;
-    switch (decode_tile(G)) {
-      case 1: return resident_workgroups<DD, 1>();
-      case 2: return resident_workgroups<DD, 2>();
-      case 4: return resident_workgroups<DD, 4>();
-      case 8: return resident_workgroups<DD, 8>();
-      default: return 512;
+    switch (tile) {
+      case 1: return resident_workgroups<DD, 1>(cap);
+      case 2: return resident_workgroups<DD, 2>(cap);
+      case 3: return resident_workgroups<DD, 3>(cap);
+      case 4: return resident_workgroups<DD, 4>(cap);
+      case 5: return resident_workgroups<DD, 5>(cap);
+      case 6: return resident_workgroups<DD, 6>(cap);
+      default: return resident_workgroups<DD, 8>(cap);   // 7 holds as many
     }
   };
   switch (D) {
@@ -773,10 +791,14 @@ int resident_for(int D, int G) {
 
 template <int D>
 int dispatch_g(const DecodeArgs& a, hipStream_t st) {
-  switch (decode_tile(a.group)) {
+  switch (a.tile) {
     case 1: return launch_decode<D, 1>(a, st);
     case 2: return launch_decode<D, 2>(a, st);
+    case 3: return launch_decode<D, 3>(a, st);
     case 4: return launch_decode<D, 4>(a, st);
+    case 5: return launch_decode<D, 5>(a, st);
+    case 6: return launch_decode<D, 6>(a, st);
+    case 7: return launch_decode<D, 7>(a, st);
     default: return launch_decode<D, 8>(a, st);
   }
 }
@@ -789,7 +811,7 @@ int gqa_decode_impl(const void* q, const void* k_cache, const void* v_cache, voi
                     const WinArgs* win = nullptr) {
   AILA_REQUIRE(q && k_cache && v_cache && out, "gqa_decode: null pointer");
   AILA_REQUIRE(B > 0 && B <= 65535 && Hq > 0 && Hkv > 0 && Hq % Hkv == 0 &&
-                   static_cast<long>(Hkv) * ((Hq / Hkv + decode_tile(Hq / Hkv) - 1) / decode_tile(Hq / Hkv)) <= 65535,
+                   static_cast<long>(Hkv) * ((Hq / Hkv + 7) / 8) <= 65535,
                "gqa_decode: bad heads/batch (B=%d Hq=%d Hkv=%d)", B, Hq, Hkv);
   AILA_REQUIRE(cached_len >= 0 && cached_len <= max_seq,
                "gqa_decode: cached_len=%d outside [0, max_seq=%d]", cached_len, max_seq);
@@ -800,7 +822,8 @@ int gqa_decode_impl(const void* q, const void* k_cache, const void* v_cache, voi
   a.out = static_cast<bf16*>(out);
   a.B = B; a.Hq = Hq; a.Hkv = Hkv; a.max_seq = max_seq; a.L = cached_len;
   a.group = Hq / Hkv;
-  a.chunks = (a.group + decode_tile(a.group) - 1) / decode_tile(a.group);
+  a.tile = decode_tile(a.group, D, pages != nullptr);
+  a.chunks = (a.group + a.tile - 1) / a.tile;
   a.seq_lens = seq_lens; a.len_bias = len_bias;
   a.k_new = static_cast<const bf16*>(k_new);
   a.v_new = static_cast<const bf16*>(v_new);
@@ -837,7 +860,7 @@ int gqa_decode_impl(const void* q, const void* k_cache, const void* v_cache, voi
     // config 1 (512 rows, 8 KV heads) takes 6.4 us in 8 splits of 64 rows
     // against 7.1 us in 4 of 128.
     const int groups = B * Hkv * a.chunks;   // workgroups per split
-    const int resident = resident_for(D, Hq / Hkv);
+    const int resident = resident_for(D, a.tile, pages != nullptr);
     int want = (resident + groups - 1) / groups;
     want = std::max(1, std::min(want, a.nsplit_max));
     a.split_len = (plan_len + want - 1) / want;
@@ -847,7 +870,12 @@ int gqa_decode_impl(const void* q, const void* k_cache, const void* v_cache, voi
     // split's start-up then covers twice the rows (B=1, Hq=16, Hkv=4,
     // D=256, L=8192: 15.0 -> 12.8 us; Hq=32, Hkv=8, D=128, L=4096: 10.1 ->
     // 9.5 us). Shorter contexts keep one chunk per wave (config 1).
-    if (a.split_len < 2 * kWaves * kChunk && plan_len >= 4096) a.split_len = 2 * kWaves * kChunk;
+    // So do ratios above 8 whose one-chunk splits would leave some of the 256 CUs
+    // two of them and some one (12 on 4 KV heads, 3000 rows: D = 128 13.0 -> 11.8
+    // us, D = 256 16.4 -> 14.0; 2048 rows, one a CU: 10.7, in two chunks 11.6).
+    const long one_chunk = static_cast<long>(groups) * ((plan_len + kWaves * kChunk - 1) / (kWaves * kChunk));
+    if (a.split_len < 2 * kWaves * kChunk && (plan_len >= 4096 || (a.chunks > 1 && one_chunk > 256)))
+      a.split_len = 2 * kWaves * kChunk;
     a.nsplit = (plan_len + a.split_len - 1) / a.split_len;
     if (a.nsplit > 1) a.part = static_cast<float*>(workspace);   // one split: direct output
   } else {

@@ -1,8 +1,7 @@
 """GPU parity of the decode entry points for any query/KV head ratio
 (the reference maps query head h to KV head h / (Hq / Hkv),
-AttentionOps.cpp:100): ratios that are not 1, 2, 4 or 8 run on the next
-larger query-head tile with the spare rows unused, ratios above 8 on
-several workgroups per KV head. Qwen3-14B (40 q / 8 kv heads) has ratio 5.
+AttentionOps.cpp:100): ratios up to 8 run on a query-head tile of their
+size, ratios above 8 on several workgroups per KV head. Qwen3-14B (40 q / 8 kv heads) has ratio 5.
 
 Tolerance: bf16 outputs within max relative error 1e-2 of the fp32 oracle.
 """
@@ -47,7 +46,7 @@ def _ws(B, Hq, D):
     (3, 2, 256, 2, 2000, True),
     (6, 2, 64, 3, 333, True),
     (7, 1, 128, 2, 100, True),      # short context: single pass with a workspace
-    (12, 2, 128, 2, 1500, True),    # two workgroups per KV head (8 + 4 heads)
+    (12, 2, 128, 2, 1500, True),    # two workgroups per KV head (6 + 6 heads)
     (16, 4, 256, 2, 3000, True),    # 64 q / 4 kv heads
     (16, 1, 128, 1, 900, False),
 ])
