@@ -859,14 +859,15 @@ __global__ __launch_bounds__(2 * kThreads, 1) void gqa_prefill_shared_kernel(
   constexpr std::integral_constant<bool, false> no{};
   auto ktile = [&](int j) __attribute__((always_inline)) { return sK[0] + (j & (NB - 1)) * C::TILE; };
   auto vtile = [&](int j) __attribute__((always_inline)) { return sV[0] + (j & (NB - 1)) * C::TILE; };
-  // V(j) between its two barriers. Blocks wholly in a wave's future are masked
-  // like the diagonal one (their P is zero).
-  auto vector = [&](int j) __attribute__((always_inline)) {
+  // V(j) between its two barriers; `live`: block j has keys this wave attends.
+  auto vector = [&](int j, auto live) __attribute__((always_inline)) {
     phase_barrier();
     const int jn = j + ahead;
     if (jn < N) issue_tile(mine + (jn & (NB - 1)) * C::TILE, kb_of(jn));
-    s_key0 = kb_of(j) * BN;
-    softmax(s_key0 + BN - 1 > start_pos + row0);
+    if constexpr (decltype(live)::value) {
+      s_key0 = kb_of(j) * BN;
+      softmax(s_key0 + BN - 1 > start_pos + row0);
+    }
     // K_{j+1} (A, two tiles issued since) or V_{j+1} (B, one) must have landed
     if (grp == 0 && jn < N) __builtin_amdgcn_s_waitcnt(vmcnt_imm<2 * C::LOADS>());
     else if (grp == 0 ? jn - 1 < N : jn < N) __builtin_amdgcn_s_waitcnt(vmcnt_imm<C::LOADS>());
@@ -879,16 +880,22 @@ __global__ __launch_bounds__(2 * kThreads, 1) void gqa_prefill_shared_kernel(
   for (int seg = nl > 0 ? 0 : 1; seg < 2; ++seg) {   // light block, heavy block
     const int end = seg == 0 ? nl : N;
     begin_segment(seg == 0 ? ql : qh);
-    if (j < end) {
+    // Blocks from jv on lie wholly in this wave's future. It does nothing in
+    // their phases: P would be zero there, but zero times a V row that is not
+    // finite is not.
+    const int jv = min(end, (seg == 0 ? 0 : nl - h0) + (start_pos + row0 + RPW - 1) / BN + 1);
+    if (j < jv) {
       matrix(no, yes, vtile(j), ktile(j));
-      vector(j);
+      vector(j, yes);
 #pragma unroll 1
-      for (++j; j < end; ++j) {
+      for (++j; j < jv; ++j) {
         matrix(yes, yes, vtile(j - 1), ktile(j));
-        vector(j);
+        vector(j, yes);
       }
       matrix(yes, no, vtile(j - 1), ktile(j));
     }
+#pragma unroll 1
+    for (; j < end; ++j) vector(j, no);
     store_segment();   // the next segment's first S follows in the same phase
   }
   phase_barrier();

@@ -4,7 +4,8 @@ rounds; key-split turns with an even number of 64-row blocks), with an odd
 number of blocks, ragged last blocks and tiles, and over a cached prefix not
 aligned to either. Rows are checked against the oracle's decode of that row over
 the rows it attends (AttentionOps.cpp:73-166 against :649-842, :2308-2507);
-bf16 outputs within 1e-2 of the row's maximum."""
+bf16 outputs within 1e-2 of the row's maximum. Rows are also checked to be
+bitwise the same when a V row outside their reach is not finite."""
 import numpy as np
 import pytest
 
@@ -73,3 +74,37 @@ def test_shared_turn(S, start, split):
     out = aila_amd.gqa_prefill_cached(_t(q), _t(k), _t(v), start, Hq, workspace=ws)
     torch.cuda.synchronize()
     _check(q, k, v, dg.bf16_to_f32(_np(out)), S, start, Hq, Hkv, max_seq)
+
+
+@pytest.mark.parametrize("S,start,Hq,row", [(3456, 0, 16, 100), (3456, 0, 16, 3455), (2047, 0, 32, 1100), (250, 2051, 16, 100),
+                                            (250, 2051, 16, 249), (500, 5003, 16, 70), (128, 3000, 16, 127)])
+def test_not_finite_v_row(S, start, Hq, row):
+    """A wave (16 query rows) reads no key block (32 rows) that lies wholly past
+    its last row, so one V row of infinities leaves every such row's bits as
+    they are without it. The rows that attend it are checked to be spoiled, so
+    that the poison is known to be read."""
+    import torch
+    import aila_amd
+    print(f"shared V row S={S} start={start} Hq={Hq} row={row}", flush=True)
+    Hkv, seed = 4, 9500 + S + row
+    q = _t(dg.normal_bf16(seed, 0, (S, Hq * D)))
+    if start:
+        n = start + S
+        k, v = (dg.normal_bf16(seed, i, (Hkv, n, D)) for i in (1, 2))
+        bad = v.copy()
+        bad[:, start + row] = 0x7F80
+        need = aila_amd.gqa_prefill_cached_workspace_size(S, start, Hq, Hkv, D)
+        assert need > 0, "planned with a key split"
+        run = lambda x: aila_amd.gqa_prefill_cached(q, _t(k), _t(x), start, Hq,  # noqa: E731
+                                                    workspace=torch.empty(need, dtype=torch.uint8, device="cuda"))
+    else:
+        k, v = (dg.normal_bf16(seed, i, (S, Hkv * D)) for i in (1, 2))
+        bad = v.copy()
+        bad[row] = 0x7F80
+        run = lambda x: aila_amd.gqa_prefill(q, _t(k), _t(x), Hq, Hkv)  # noqa: E731
+    clean, got = _np(run(v)), _np(run(bad))
+    reach = (start + row) // 32 * 32                        # first key of the poisoned block
+    free = [r for r in range(S) if start + r // 16 * 16 + 15 < reach]
+    assert free and free[-1] >= row - 48
+    assert np.array_equal(got[free], clean[free])
+    assert not np.isfinite(dg.bf16_to_f32(got[row:])).any()
