@@ -760,15 +760,20 @@ int resident_workgroups(int max_per_cu) {
   return std::min(known >> 16, max_per_cu) * (known & 0xffff);
 }
 
-// The plan's workgroups for one round. Three a CU stream no faster than two at
-// D = 128 (tiles 3 and 4: B = 8, 4 KV heads, 16384 rows 5% slower; tile 6 over two
-// workgroups a KV head 54 / 39 us), and the paged kernel, with up to 10 registers
-// more, would not hold them all at once (tile 2, 16384 rows: 12% slower; tile 6:
-// 40 / 31 us); tile 1 and 2 over a contiguous cache measured within 3% either way.
-// At D = 64 tiles 3 and 5 to 7 take three, as tile 8 does (paged tile 3 at 16384
-// rows 13% slower otherwise); 1, 2 and 4 measured up to 10% faster with all theirs.
-int resident_for(int D, int tile, bool paged) {
-  const int cap = D == 64 ? (tile == 3 || tile > 4 ? 3 : 8) : D == 128 && (paged || tile >= 3) ? 2 : 8;
+// The plan's workgroups for one round: the same for a contiguous and a paged
+// cache, whose results on the same rows are the same bits only if the rows are
+// split alike. Tiles 1 to 4 at D = 128 take all their occupancy: capped at two a
+// CU a contiguous cache loses more than a paged one gains (120 shapes, 1-32
+// sequences of 1000-32768 rows, all / two a CU: tile 1 geometric mean 5% slower,
+// B = 22, 1 KV head, 31744 rows 57.9 / 70.0 us; tile 2 5%; tile 3 4%, B = 14, 2 KV
+// heads, 25728 rows 62.4 / 73.4; tile 4 2%, B = 5, 8 KV heads, 6656 rows 27.9 /
+// 32.8; paged, tile 2 6% faster, the others within 2%). Tiles 5 and 6 stream no
+// faster with three a CU than with two there (tile 6 over two workgroups a KV head
+// 54 / 39 us, paged 40 / 31). At D = 64 tiles 3 and 5 to 7 take three, as tile 8
+// does (paged tile 3 at 16384 rows 13% slower otherwise); 1, 2 and 4 measured up to
+// 10% faster with all theirs.
+int resident_for(int D, int tile) {
+  const int cap = D == 64 ? (tile == 3 || tile > 4 ? 3 : 8) : D == 128 && tile > 4 ? 2 : 8;
   auto pick = [&](auto d_tag) -> int {
     constexpr int DD = decltype(d_tag)::value;
     switch (tile) {
@@ -860,7 +865,7 @@ int gqa_decode_impl(const void* q, const void* k_cache, const void* v_cache, voi
     // config 1 (512 rows, 8 KV heads) takes 6.4 us in 8 splits of 64 rows
     // against 7.1 us in 4 of 128.
     const int groups = B * Hkv * a.chunks;   // workgroups per split
-    const int resident = resident_for(D, a.tile, pages != nullptr);
+    const int resident = resident_for(D, a.tile);
     int want = (resident + groups - 1) / groups;
     want = std::max(1, std::min(want, a.nsplit_max));
     a.split_len = (plan_len + want - 1) / want;

@@ -140,3 +140,25 @@ def test_paged_rejects_bad_arguments():
     pages = torch.zeros((4, 2, 32, 128), dtype=torch.bfloat16, device="cuda")
     with pytest.raises(aila_amd.AilaHipError):
         aila_amd.gqa_decode_paged(q, pages, pages, table, sl, 4 * 32 + 1)  # max_len beyond the table
+
+
+@pytest.mark.parametrize("B,Hkv,D,G,L", [(32, 8, 128, 1, 2100), (32, 8, 128, 2, 4096), (21, 2, 128, 1, 8128), (12, 8, 128, 3, 2304),
+                                         (16, 8, 128, 4, 2000), (10, 8, 128, 7, 2048), (8, 4, 128, 14, 2048),
+                                         (16, 8, 64, 3, 2048), (16, 8, 256, 2, 2048)])
+def test_paged_equals_contiguous_where_the_device_is_full(B, Hkv, D, G, L):
+    """Enough sequences and KV heads that the workgroups the device holds, and
+    not the rows, set the number of splits."""
+    import torch
+    import aila_amd
+    print(f"paged full device B={B} Hkv={Hkv} D={D} G={G} L={L}", flush=True)
+    page, mp = 64, (L + 63) // 64
+    g = torch.Generator(device="cuda").manual_seed(B + D + G)
+    q = torch.empty((B, Hkv * G, D), device="cuda", dtype=torch.bfloat16).normal_(generator=g)
+    pk, pv = (torch.empty((B * mp, Hkv, page, D), device="cuda", dtype=torch.bfloat16).normal_(generator=g) for _ in range(2))
+    table = torch.from_numpy(np.random.default_rng(G).permutation(B * mp).astype(np.int32)).view(B, mp).cuda()
+    kc, vc = (p[table.long()].transpose(1, 2).reshape(B, Hkv, mp * page, D).contiguous() for p in (pk, pv))
+    lens = (L - torch.arange(B, dtype=torch.int32) % 7 * 100).cuda()
+    ws = torch.empty(aila_amd.gqa_decode_workspace_size(B, Hkv * G, D), dtype=torch.uint8, device="cuda")
+    got = aila_amd.gqa_decode_paged(q, pk, pv, table, lens, L, workspace=ws)
+    ref = aila_amd.gqa_decode(q, kc, vc, L, workspace=ws, seq_lens=lens)
+    assert torch.equal(got, ref)
