@@ -569,11 +569,10 @@ __global__ __launch_bounds__(kThreads) void gqa_decode_split_kernel(
 // so its record reads are independent and issued together; the P partial
 // sums meet in LDS.
 // CS workgroups per head, each for D / CS dims: with few heads (a single
-// sequence) one workgroup per head leaves most CUs idle and walks its records in
-// several rounds of loads (16 heads, 128 records each, D = 256: merge 6.0 -> 3.6 us).
-// The decode call at 8192 rows, D = 256, one workgroup a head against 64 dims
-// each: 16 heads 14.4 -> 11.9 us, 32 18.1 -> 17.4, 64 27.1 / 27.0, 128 47.5 / 48.2;
-// so up to 32 heads.
+// sequence) and more records than one workgroup reads in one round of loads, one
+// workgroup per head leaves most CUs idle and walks its records in several rounds
+// (16 heads, 128 records each, D = 256: merge 6.0 -> 3.6 us). The launch's rule
+// has both sides measured.
 template <int D, bool WIN = false, int CS = 1>
 __global__ __launch_bounds__(256) void gqa_decode_merge_kernel(
     const float* __restrict__ part, bf16* __restrict__ out, int Hq, int L,
@@ -703,8 +702,14 @@ int launch_decode(const DecodeArgs& a, hipStream_t st) {
   }
   if (a.part) {
     const bool gated = a.prep.q_stride > 0 && a.prep.apply_gate;
-    constexpr int CS = D / 64;   // 64 dims a workgroup (see the kernel)
-    if (!win && CS > 1 && a.Hq * a.B <= 32)
+    // 64 dims a workgroup for up to 32 heads (the decode call at 8192 rows, D =
+    // 256, one workgroup a head against 64 dims each: 16 heads 14.4 -> 11.9 us, 32
+    // 18.1 -> 17.4, 64 27.1 / 27.0, 128 47.5 / 48.2) of more records than the 256
+    // threads' one round of eight loads (D = 256: 38 records 10.6 -> 10.2, 34 9.8 ->
+    // 9.3, 30 8.4 / 8.5, 6 9.4 / 9.9; D = 128: 65 11.4 -> 10.7, 48 10.2 / 10.2, 5
+    // 7.5 / 7.8).
+    constexpr int CS = D / 64, kOneRound = 8 * (256 / (D / 4));
+    if (!win && CS > 1 && a.Hq * a.B <= 32 && a.nsplit > kOneRound)
       hipLaunchKernelGGL((gqa_decode_merge_kernel<D, false, CS>), dim3(a.Hq, a.B, CS), dim3(256), 0, st, a.part, a.out,
                          a.Hq, a.L, a.seq_lens, a.len_bias, a.split_len, a.nsplit, a.nsplit_max,
                          gated ? a.q + D : nullptr, a.prep.q_stride, a.win);

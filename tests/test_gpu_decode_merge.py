@@ -1,4 +1,5 @@
 """GPU parity of the split-K decode's merge on both sides of the head count
+and of the number of records (32 at D = 256, 64 at D = 128: splits of 128 rows)
 where it changes from several workgroups per head (64 dims each) to one,
 against the CPU oracle (AttentionOps.cpp:73-166). bf16 outputs within 1e-2 of
 the tensor maximum."""
@@ -21,7 +22,7 @@ def _t(x):
 def test_merge_either_side_of_32_heads(B, Hq, Hkv, D):
     import torch
     import aila_amd
-    for L in (257, 1100, 4500):
+    for L in (257, 1100, 4096, 4097, 8192, 8193):
         seed = 7100 + 31 * B + D + L
         q = dg.normal_bf16(seed, 0, (B, Hq, D))
         k, v = (dg.normal_bf16(seed, i, (B, Hkv, L, D)) for i in (1, 2))
