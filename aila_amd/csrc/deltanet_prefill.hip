@@ -27,9 +27,10 @@
 // output-only products (Q S, P D) use single bf16 (S as hi + lo in the layer).
 //
 // Kernel 1 (deltanet_chunk_prep_kernel): one workgroup per (chunk, key head,
-//   sequence) forms what the recurrence needs and S does not enter: K, Q,
-//   K K^T and Q K^T once for the key head, then To and P for each of its
-//   value heads (four waves per value head).
+//   sequence), or several that share the key head's value heads where the grid
+//   is small, forms what the recurrence needs and S does not enter: K, Q,
+//   K K^T and Q K^T once, then To and P for each of its value heads (four waves
+//   per value head).
 // Kernel 2 (deltanet_chunk_scan_kernel): one 8-wave workgroup per (slab of 16
 //   NT columns of dv, value head, sequence) walks the chunks in order with
 //   its state slab in registers of four "state" waves, while four "output"
@@ -170,9 +171,9 @@ __host__ __device__ __forceinline__ size_t key_rec_offset(int b, int hk, int c, 
 // an output far below sqrt(eps)): Q K^T takes Q_hi K_hi + Q_hi K_lo +
 // Q_lo K_hi and the scan's Q S takes S as hi + lo.
 //
-// GP value heads are formed at a time by 4 waves each; a key head with more
-// runs in passes. Its conv, norms and two products are then formed once (one
-// workgroup per value head repeated them), and GP heads' serial inversions are
+// A workgroup takes `per` of its key head's value heads (see launch_prep), GP at
+// a time by 4 waves each; more run in passes. The conv, norms and two products
+// are formed once a workgroup, and GP heads' serial inversions are
 // in flight side by side: the kernel is bound by those dependent chains (about
 // 14 us at one chunk) and, over many chunks, by its ~120 MB of traffic at
 // T = 4096, Hk = 16, Hv = 32 (44 us, 2.7 TB/s; two workgroups of 67 KiB a CU).
@@ -180,7 +181,7 @@ template <bool kLo, int GP>
 __global__ __launch_bounds__(kHeadThreads * GP, GP == 2 ? 4 : GP == 1 ? 2 : GP) void deltanet_chunk_prep_kernel(
     const bf16* __restrict__ q, const bf16* __restrict__ k, ConvIn cv, const bf16* __restrict__ a,
     const bf16* __restrict__ bg, int ab_stride, const bf16* __restrict__ dt_bias, const float* __restrict__ A_log,
-    unsigned char* __restrict__ ws, int T, int Hk, int Hv, float eps) {
+    unsigned char* __restrict__ ws, int T, int Hk, int Hv, int per, float eps) {
   using R = ChunkRec;
   using RK = KeyRec<kLo>;
   constexpr int kThr = kHeadThreads * GP, NW = 4 * GP;
@@ -196,9 +197,11 @@ __global__ __launch_bounds__(kHeadThreads * GP, GP == 2 ? 4 : GP == 1 ? 2 : GP) 
   unsigned char* const sKl = smem + (kLo ? 2 * kTile : 0);
   unsigned char* const sQl = smem + (kLo ? 3 * kTile : 0);
 
-  const int c = blockIdx.x, hk = blockIdx.y, b = blockIdx.z;
+  const int c = blockIdx.x, hk = static_cast<int>(blockIdx.y) % Hk, b = blockIdx.z;
   const int nch = (T + kC - 1) / kC;
-  const int G = Hv / Hk;
+  // value heads of this workgroup: hv0 .. hv0 + nv - 1
+  const int share = static_cast<int>(blockIdx.y) / Hk;
+  const int hv0 = hk * (Hv / Hk) + share * per, nv = min(per, Hv / Hk - share * per);
   const int t0 = c * kC;
   const int n = min(kC, T - t0);
   const int tid = threadIdx.x, lane = tid & 63;
@@ -210,7 +213,7 @@ __global__ __launch_bounds__(kHeadThreads * GP, GP == 2 ? 4 : GP == 1 ? 2 : GP) 
   // gates of this chunk and one value head (one wave): beta, g, prefix sum G
   auto gates = [&](int pass) __attribute__((always_inline)) {
     if (w4 != 0) return;
-    const int hv = hk * G + min(pass * GP + grp, G - 1);
+    const int hv = hv0 + min(pass * GP + grp, nv - 1);
     float beta = 0.f, g = 0.f;
     if (lane < n) {
       const size_t gi = (static_cast<size_t>(b) * T + t0 + lane) * ab_stride + hv;
@@ -389,8 +392,8 @@ __global__ __launch_bounds__(kHeadThreads * GP, GP == 2 ? 4 : GP == 1 ? 2 : GP) 
     ss += __shfl_xor(ss, 2);
     if (part == 0) (it < 256 ? sIk : sIq)[r] = 1.0f / sqrtf(ss + eps);
   }
-  // ---- 4. key-head record: K tile image(s), Q in register order ------------------
-  for (int o = tid; o < kTile / 16; o += kThr) {
+  // ---- 4. key-head record (first share): K tile image(s), Q in register order -----
+  for (int o = tid; share == 0 && o < kTile / 16; o += kThr) {
     __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(sK + o * 16), reinterpret_cast<u32x4*>(krec + RK::kK) + o);
     if constexpr (kLo)
       __builtin_nontemporal_store(*reinterpret_cast<const u32x4*>(sKl + o * 16), reinterpret_cast<u32x4*>(krec + RK::kKLo) + o);
@@ -408,9 +411,9 @@ __global__ __launch_bounds__(kHeadThreads * GP, GP == 2 ? 4 : GP == 1 ? 2 : GP) 
 
   float* const sA = reinterpret_cast<float*>(smem + kRaw + grp * 2 * kTri);
   float* const sT = sA + kTri / 4;
-  for (int pass = 0; pass * GP < G; ++pass) {
-    const bool live = pass * GP + grp < G;
-    const int hv = hk * G + min(pass * GP + grp, G - 1);
+  for (int pass = 0; pass * GP < nv; ++pass) {
+    const bool live = pass * GP + grp < nv;
+    const int hv = hv0 + min(pass * GP + grp, nv - 1);
     unsigned char* rec = ws + ((static_cast<size_t>(b) * Hv + hv) * nch + c) * R::kBytes;
     // ---- 5. A (LDS, packed tiles) and P (register order) with this head's gates --
 #pragma unroll
@@ -533,7 +536,7 @@ __global__ __launch_bounds__(kHeadThreads * GP, GP == 2 ? 4 : GP == 1 ? 2 : GP) 
         __builtin_nontemporal_store(lo, reinterpret_cast<u32x4*>(rec + R::kTLo) + (w4 * 2 + ks) * 64 + lane);
       }
     }
-    if ((pass + 1) * GP < G) {
+    if ((pass + 1) * GP < nv) {
       __syncthreads();   // the gates and A of this pass are no longer read
       gates(pass + 1);
       __syncthreads();
@@ -996,12 +999,25 @@ template <bool kLo>
 void launch_prep(const bf16* q, const bf16* k, const ConvIn& cv, const bf16* a, const bf16* b, int ab_stride,
                  const bf16* dt_bias, const float* A_log, unsigned char* records, int B, int T, int Hk, int Hv,
                  float eps, hipStream_t st) {
+  // Value heads per workgroup: all of the key head's, more than four in passes, or
+  // shares of two (each forms the key head's tiles and products again). Shares are
+  // faster while each finds one of the 256 CUs, and where they replace passes until
+  // the whole key heads fill 5/8 of the CUs by themselves. Whole key head / shares,
+  // us at n workgroups of whole key heads: recurrence, ratio 16, n = 1 46.0 / 16.6,
+  // 64 81.8 / 56.8, 128 94.5 / 79.6, 192 115.8 / 112.3, 256 142.4 / 146.6; ratio 4, 1
+  // 19.7 / 16.4, 128 55.5 / 52.5; layer, ratio 16, 1 55.5 / 26.8, 128 134.7 / 127.8,
+  // 192 171.7 / 177.4; ratio 8, 128 88.2 / 82.8, 192 111.1 / 114.2, 512 224 / 241;
+  // ratio 4, 128 73.4 / 71.5, 192 94.4 / 97.0; ratio 3, 128 69.5 / 69.8, 160 44.7 / 50.0.
+  const int G = Hv / Hk, nch = (T + kC - 1) / kC;
+  const long whole = static_cast<long>(nch) * Hk * B;
+  const int per = whole * ((G + 1) / 2) <= 256 || (G > 4 && whole < 160) ? std::min(G, 2) : G;
   auto go = [&](auto gp) {
     constexpr int GP = decltype(gp)::value;
-    hipLaunchKernelGGL((deltanet_chunk_prep_kernel<kLo, GP>), dim3((T + kC - 1) / kC, Hk, B), dim3(kHeadThreads * GP),
-                       0, st, q, k, cv, a, b, ab_stride, dt_bias, A_log, records, T, Hk, Hv, eps);
+    hipLaunchKernelGGL((deltanet_chunk_prep_kernel<kLo, GP>), dim3(nch, Hk * ((G + per - 1) / per), B),
+                       dim3(kHeadThreads * GP), 0, st, q, k, cv, a, b, ab_stride, dt_bias, A_log, records, T, Hk, Hv,
+                       per, eps);
   };
-  switch (Hv / Hk) {
+  switch (per) {
     case 1: go(std::integral_constant<int, 1>{}); break;
     case 2: go(std::integral_constant<int, 2>{}); break;
     case 3: go(std::integral_constant<int, 3>{}); break;

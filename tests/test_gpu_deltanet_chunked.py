@@ -1,6 +1,7 @@
 """GPU parity of the chunked DeltaNet prefill over the forms its dispatch
 distinguishes: value heads per key head (one prep workgroup forms 1-4 of them
-at a time, more in passes), column slabs of the scan (16, 32 or 64 columns by
+at a time, more in passes; on small grids several share a key head, two value
+heads each), column slabs of the scan (16, 32 or 64 columns by
 the number of heads) and chunk counts around its two- and three-chunk
 rotations, against the sequential oracle recurrence
 (run_linear_delta_host, Qwen35HybridTextBackend.cpp:1640-1798).
@@ -81,6 +82,14 @@ def test_layer_matches_oracle(B, Hk, Hv, T):
     assert _rel(st.cpu().numpy(), want_S) <= STATE_TOL
     assert _rel(_bf(out), dg.bf16_to_f32(want_o)) <= OUT_TOL
     assert np.array_equal(cs.cpu().numpy(), want_cs)
+
+
+@pytest.mark.parametrize("B,G", [(64, 3), (65, 3), (64, 4), (65, 4), (79, 5), (80, 5), (79, 8), (80, 8)])
+def test_prep_either_side_of_its_rule(B, G):
+    # two chunks a sequence: shares of two value heads up to 256 workgroups (more than
+    # four heads: below 160 of whole key heads), the last one ragged; then whole key heads
+    test_recurrence_matches_oracle(B, 1, G, 65)
+    test_layer_matches_oracle(B, 1, G, 65)
 
 
 @pytest.mark.parametrize("wide", [False, True])
