@@ -746,23 +746,25 @@ int decode_tile(int g, int D, bool paged) {
 // extra round pays the workgroup start-up latency and a partial tail).
 // The per-device value is idempotent, so concurrent first calls may both
 // compute it; the atomic makes the publication race-free.
+struct Residency { int per_cu, cus; };
 template <int D, int G>
-int resident_workgroups(int max_per_cu) {
+Residency resident_workgroups(int max_per_cu) {
   constexpr int kMaxDev = 64;
+  constexpr Residency kUnknown{2, 256};
   static std::atomic<int> cache[kMaxDev];   // workgroups per CU << 16 | CUs
   int dev = 0;
-  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) return 512;
+  if (hipGetDevice(&dev) != hipSuccess || dev < 0 || dev >= kMaxDev) return kUnknown;
   int known = cache[dev].load(std::memory_order_relaxed);
   if (known <= 0) {
     int per_cu = 0, cus = 0;
     if (hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, gqa_decode_split_kernel<D, G>, kThreads, 0) !=
             hipSuccess ||
         hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess || per_cu <= 0 || cus <= 0)
-      return 512;
+      return kUnknown;
     known = per_cu << 16 | cus;
     cache[dev].store(known, std::memory_order_relaxed);
   }
-  return std::min(known >> 16, max_per_cu) * (known & 0xffff);
+  return {std::min(known >> 16, max_per_cu), known & 0xffff};
 }
 
 // The plan's workgroups for one round: the same for a contiguous and a paged
@@ -781,11 +783,11 @@ int resident_workgroups(int max_per_cu) {
 // average there (600 calls), and where they make twice as many short splits as one
 // round takes they lose up to 20% (B = 30, 8 KV heads, ratio 12, 512 of 1024 rows
 // 47 / 61 us; B = 15, ratio 6, 2073 of 2304 rows 52 / 61).
-int resident_for(int D, int tile, bool wide_window) {
+Residency resident_for(int D, int tile, bool wide_window) {
   const int cap = D == 64    ? (tile == 3 || tile > 4 ? 3 : 8)
                   : D == 128 ? (tile > 4 ? 2 : 8)
                              : (wide_window ? 1 : 8);
-  auto pick = [&](auto d_tag) -> int {
+  auto pick = [&](auto d_tag) -> Residency {
     constexpr int DD = decltype(d_tag)::value;
     switch (tile) {
       case 1: return resident_workgroups<DD, 1>(cap);
@@ -801,7 +803,7 @@ int resident_for(int D, int tile, bool wide_window) {
     case 64: return pick(std::integral_constant<int, 64>{});
     case 128: return pick(std::integral_constant<int, 128>{});
     case 256: return pick(std::integral_constant<int, 256>{});
-    default: return 512;
+    default: return {2, 256};
   }
 }
 
@@ -876,8 +878,8 @@ int gqa_decode_impl(const void* q, const void* k_cache, const void* v_cache, voi
     // config 1 (512 rows, 8 KV heads) takes 6.4 us in 8 splits of 64 rows
     // against 7.1 us in 4 of 128.
     const int groups = B * Hkv * a.chunks;   // workgroups per split
-    const int resident = resident_for(D, a.tile, a.win.window > 0 && a.group > 4);
-    int want = (resident + groups - 1) / groups;
+    const Residency resident = resident_for(D, a.tile, a.win.window > 0 && a.group > 4);
+    int want = (resident.per_cu * resident.cus + groups - 1) / groups;
     want = std::max(1, std::min(want, a.nsplit_max));
     a.split_len = (plan_len + want - 1) / want;
     a.split_len = ((a.split_len + kWaves * kChunk - 1) / (kWaves * kChunk)) * (kWaves * kChunk);
@@ -886,12 +888,19 @@ int gqa_decode_impl(const void* q, const void* k_cache, const void* v_cache, voi
     // split's start-up then covers twice the rows (B=1, Hq=16, Hkv=4,
     // D=256, L=8192: 15.0 -> 12.8 us; Hq=32, Hkv=8, D=128, L=4096: 10.1 ->
     // 9.5 us). Shorter contexts keep one chunk per wave (config 1).
-    // So do ratios above 8 whose one-chunk splits would leave some of the 256 CUs
-    // two of them and some one (12 on 4 KV heads, 3000 rows: D = 128 13.0 -> 11.8
-    // us, D = 256 16.4 -> 14.0; 2048 rows, one a CU: 10.7, in two chunks 11.6).
-    const long one_chunk = static_cast<long>(groups) * ((plan_len + kWaves * kChunk - 1) / (kWaves * kChunk));
-    if (a.split_len < 2 * kWaves * kChunk && (plan_len >= 4096 || (a.chunks > 1 && one_chunk > 256)))
-      a.split_len = 2 * kWaves * kChunk;
+    // So do ratios above 8 whose one-chunk splits are more than the CUs (12 on 4 KV
+    // heads, 3000 rows: D = 128 13.0 -> 11.8 us, D = 256 16.4 -> 14.0; 2048 rows, one
+    // a CU: 10.7, in two chunks 11.6), unless those run at once, at most two a CU,
+    // and the longer ones are more than the CUs too (B = 9, 16 on 4, 399 rows, D =
+    // 128: 504 against 288 workgroups, 15.8 / 16.9; B = 6, 14 on 8, 352 rows: 576
+    // against 288, 20.2 / 17.8).
+    auto workgroups = [&](int chunks) {   // in splits of `chunks` 16-row chunks per wave
+      const int rows = chunks * kWaves * kChunk;
+      return static_cast<long>(groups) * ((plan_len + rows - 1) / rows);
+    };
+    const long one = workgroups(1), cus = resident.cus;
+    const bool unequal = a.chunks > 1 && one > cus && (one > std::min(resident.per_cu, 2) * cus || workgroups(2) <= cus);
+    if (a.split_len < 2 * kWaves * kChunk && (plan_len >= 4096 || unequal)) a.split_len = 2 * kWaves * kChunk;
     a.nsplit = (plan_len + a.split_len - 1) / a.split_len;
     if (a.nsplit > 1) a.part = static_cast<float*>(workspace);   // one split: direct output
   } else {

@@ -49,6 +49,9 @@ def _ws(B, Hq, D):
     (12, 2, 128, 2, 1500, True),    # two workgroups per KV head (6 + 6 heads)
     (16, 4, 256, 2, 3000, True),    # 64 q / 4 kv heads
     (16, 1, 128, 1, 900, False),
+    (16, 4, 128, 9, 399, True),     # splits of 64 rows: 504 workgroups, at once
+    (14, 8, 128, 6, 352, True),     # of 128: 576 of 64 would not run at once
+    (12, 4, 128, 1, 3000, True),    # of 128: 192 workgroups, one to a CU
 ])
 def test_decode_any_group(G, Hkv, D, B, L, split):
     import torch
