@@ -778,15 +778,9 @@ Residency resident_workgroups(int max_per_cu) {
 // faster with three a CU than with two there (tile 6 over two workgroups a KV head
 // 54 / 39 us, paged 40 / 31). At D = 64 tiles 3 and 5 to 7 take three, as tile 8
 // does (paged tile 3 at 16384 rows 13% slower otherwise); 1, 2 and 4 measured up to
-// 10% faster with all theirs. The window kernel of ratios above 4
-// keeps one a CU at D = 256, as tile 8 holds: the smaller tiles' two gain nothing on
-// average there (600 calls), and where they make twice as many short splits as one
-// round takes they lose up to 20% (B = 30, 8 KV heads, ratio 12, 512 of 1024 rows
-// 47 / 61 us; B = 15, ratio 6, 2073 of 2304 rows 52 / 61).
-Residency resident_for(int D, int tile, bool wide_window) {
-  const int cap = D == 64    ? (tile == 3 || tile > 4 ? 3 : 8)
-                  : D == 128 ? (tile > 4 ? 2 : 8)
-                             : (wide_window ? 1 : 8);
+// 10% faster with all theirs.
+Residency resident_for(int D, int tile) {
+  const int cap = D == 64 ? (tile == 3 || tile > 4 ? 3 : 8) : D == 128 && tile > 4 ? 2 : 8;
   auto pick = [&](auto d_tag) -> Residency {
     constexpr int DD = decltype(d_tag)::value;
     switch (tile) {
@@ -878,7 +872,14 @@ int gqa_decode_impl(const void* q, const void* k_cache, const void* v_cache, voi
     // config 1 (512 rows, 8 KV heads) takes 6.4 us in 8 splits of 64 rows
     // against 7.1 us in 4 of 128.
     const int groups = B * Hkv * a.chunks;   // workgroups per split
-    const Residency resident = resident_for(D, a.tile, a.win.window > 0 && a.group > 4);
+    Residency resident = resident_for(D, a.tile);
+    // The window kernel of ratios above 4 at D = 256: where two workgroups a CU
+    // would make three splits or fewer, one a CU sets the number, so that the splits
+    // run at once (25 sequences, 12 on 8 KV heads, 976 rows: 2 splits of 400
+    // workgroups 34.1 us, 1 24.3; B = 9, 17 on 8, 6354 rows, window 1579: 3 of 216
+    // 80.7, 2 71.4). More splits take two a CU (B = 4, 11 on 8, window 4462: 8 of 64
+    // 45.2, 4 71.9; B = 37, 9 on 2, window 572: 4 of 148 24.2, 2 28.6).
+    if (a.win.window > 0 && a.group > 4 && D == 256 && 3 * groups > 2 * resident.cus) resident.per_cu = 1;
     int want = (resident.per_cu * resident.cus + groups - 1) / groups;
     want = std::max(1, std::min(want, a.nsplit_max));
     a.split_len = (plan_len + want - 1) / want;
