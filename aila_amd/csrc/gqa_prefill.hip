@@ -977,8 +977,17 @@ bool shared_tiles(int S, int start_pos, int Hq) {
 }
 // ... and a key-split one, where both kernels launch the same workgroups as long
 // as 128-row blocks pad no more than 64-row ones do (S = 250 over 7900 rows 66 ->
-// 57 us, 512 over 4096 62 -> 57; 300 over 16000, five 64-row blocks, 165 / 192).
-bool shared_split(int S) { return (S + 63) / 64 % 2 == 0; }
+// 57 us, 512 over 4096 62 -> 57; 300 over 16000, five 64-row blocks, 165 / 192). But
+// the other kernel's walk a light and a heavy block, these one block each: in a
+// single round of the device the last block must not see more than three times the
+// first one's keys (2 heads, S = 5084 over 240 rows 70 / 95, 8131 over 775 121 / 161,
+// 1134 over 187 28.9 / 31.5; below three times 2% slower at most, over 600 shapes).
+// Further workgroups even it out (4 heads, S = 1730 over 702 56 / 49, 280 workgroups).
+bool shared_split(int S, int start_pos, int Hq, int nz) {
+  const int n64 = (S + 63) / 64;
+  const int first = (start_pos + std::min(S, 64) - 1) / 32 + 1, last = (start_pos + S - 1) / 32 + 1;
+  return n64 % 2 == 0 && (last <= 3 * first || n64 / 2 * Hq * nz > prefill_resident<256>());
+}
 
 template <int D, int RPW, int BN>
 int launch_prefill(const bf16* q, const bf16* k, const bf16* v, int kv_row_stride,
@@ -1004,7 +1013,7 @@ int launch_prefill(const bf16* q, const bf16* k, const bf16* v, int kv_row_strid
                        Hq * D, S, start_pos, Hkv, Hq / Hkv, scale_log2, split ? nullptr : k_cache,
                        split ? nullptr : v_cache, split ? 0 : cache_pos, max_seq, part);
   };
-  const bool shared = D == 256 && (part != nullptr ? shared_split(S) : shared_tiles(S, start_pos, Hq));
+  const bool shared = D == 256 && (part != nullptr ? shared_split(S, start_pos, Hq, nz) : shared_tiles(S, start_pos, Hq));
   if constexpr (D == 256) {
     const int nb = (S + 2 * C::BM - 1) / (2 * C::BM);
     if (shared && part == nullptr) go(gqa_prefill_shared_kernel<D, RPW, BN, false>, dim3((nb + 1) / 2, Hq));

@@ -56,10 +56,11 @@ def test_shared_prefill(S, Hq, Hkv, scale):
 
 
 @pytest.mark.parametrize("split", [True, False])
-@pytest.mark.parametrize("S,start", [(65, 777), (128, 3000), (250, 2051), (500, 5003), (2048, 101)])
+@pytest.mark.parametrize("S,start", [(65, 777), (128, 3000), (250, 2051), (500, 5003), (710, 250), (711, 250), (2048, 101)])
 def test_shared_turn(S, start, split):
     """Turns over a cached prefix with the key split (S = 2048: none planned) and
-    without; NaN past the rows any query attends."""
+    without; 710 and 711 tokens over 250 rows lie on both sides of three times the
+    first block's keys; NaN past the rows any query attends."""
     import torch
     import aila_amd
     Hq, Hkv = (32, 4) if S == 2048 else (16, 4)
