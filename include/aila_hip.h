@@ -327,7 +327,10 @@ int aila_hip_deltanet_decode(const void* q, const void* k, const void* v,
  * key head as aila_hip_deltanet_decode) run the general-shape kernel, the
  * role of the reference's generic fallback (:1168-1304), followed by a
  * ring-rewrite launch; conv_state is then [B, K-1, ch] and arrivals is
- * ignored, as it is for Hv / Hk = 3.
+ * ignored, as it is for Hv / Hk = 3. The tuned kernels need conv_w, z and out
+ * 8-byte aligned, z_stride a multiple of 4, norm_w and state 16-byte aligned;
+ * of calls that are not, Hv / Hk = 3 runs the general-shape kernel (slower:
+ * 31.5 against 12.0 us at B = 8, Hk = 16) and the others are refused.
  *   arrivals  optional device uint32[B*Hk], zero before the first call and
  *             left zero by every call: with it (and Hv > Hk) the layer runs
  *             one workgroup per value head instead of one per key head (the

@@ -119,3 +119,61 @@ def test_layer_decode_three_value_heads(B, Hk, wide):
     assert _rel(np.stack([_bf(o) for o in outs], axis=1), dg.bf16_to_f32(want_o)) <= OUT_TOL
     assert np.array_equal(cs.cpu().numpy(), want_cs)
     assert arr is None or (arr == 7).all().item()
+
+
+def _three_heads(B, Hk, pad):
+    """One layer step with three value heads to a key head; z rows `pad` elements apart."""
+    Hv, seed = 3 * Hk, 43500 + B
+    ch = 2 * Hk * D + Hv * D
+    x = dict(qkv=dg.normal_bf16(seed, 0, (B, 1, ch)), z=dg.normal_bf16(seed, 1, (B, 1, Hv * D)),
+             a=dg.normal_bf16(seed, 2, (B, 1, Hv)), b=dg.normal_bf16(seed, 3, (B, 1, Hv)),
+             w=dg.normal_bf16(seed, 4, (ch, 4), std=0.5), ring=dg.normal(seed, 5, B * 3 * ch).reshape(B, 3, ch),
+             norm=1.0 + dg.normal(seed, 7, D, std=0.1), S0=dg.normal(seed, 6, B * Hv * D * D, std=0.1).reshape(B, Hv, D, D))
+    zw = np.zeros((B, Hv * D + pad), np.uint16)
+    zw[:, :Hv * D] = x["z"][:, 0]
+    return x, Hv, ch, _t(zw)[:, :Hv * D]
+
+
+def test_layer_decode_three_value_heads_unaligned_z_rows():
+    """z rows a number of elements apart that is no multiple of 4: the general
+    kernel takes the call."""
+    import torch
+    import aila_amd
+    B, Hk = 3, 2
+    x, Hv, _, z = _three_heads(B, Hk, 2)
+    assert z.stride(0) % 4 == 2
+    print("deltanet_layer_decode three value heads, unaligned z rows", flush=True)
+    st, cs = _t(x["S0"]), _t(x["ring"])
+    out = aila_amd.deltanet_layer_decode(_t(x["qkv"][:, 0]), z, _t(x["a"][:, 0]), _t(x["b"][:, 0]), _t(x["w"]), cs, 1,
+                                         _t(x["norm"]), st, Hk)
+    torch.cuda.synchronize()
+    want_o, want_S, want_cs = oracle.deltanet_layer(x["qkv"], x["z"], x["a"], x["b"], x["w"], x["ring"], 1, x["norm"],
+                                                   x["S0"], B, 1, Hk, Hv, D, D, fast=True)
+    assert _rel(st.cpu().numpy(), want_S) <= STATE_TOL
+    assert _rel(_bf(out), dg.bf16_to_f32(want_o)[:, 0]) <= OUT_TOL
+    assert np.array_equal(cs.cpu().numpy(), want_cs)
+
+
+def test_layer_decode_three_value_heads_ignores_arrivals_address():
+    """The array is ignored for this ratio, its alignment too: the same kernel
+    runs, so the same bits come out."""
+    import torch
+    import aila_amd
+    B, Hk = 2, 2
+    x, Hv, ch, z = _three_heads(B, Hk, 0)
+    t = {k: _t(x[k][:, 0]) for k in ("qkv", "a", "b")}
+    w, norm = _t(x["w"]), _t(x["norm"])
+    arr = torch.full((4 * B * Hk + 4,), 7, dtype=torch.uint8, device="cuda")
+    res = []
+    for address in (None, arr.data_ptr() + 1):
+        print(f"deltanet_layer_decode three value heads, arrivals at {address}", flush=True)
+        st, cs, out = _t(x["S0"]), _t(x["ring"]), torch.empty((B, Hv * D), dtype=torch.bfloat16, device="cuda")
+        rc = aila_amd.lib().aila_hip_deltanet_layer_decode(
+            t["qkv"].data_ptr(), ch, z.data_ptr(), Hv * D, t["a"].data_ptr(), t["b"].data_ptr(), Hv, w.data_ptr(),
+            cs.data_ptr(), 0, None, None, None, norm.data_ptr(), st.data_ptr(), out.data_ptr(), B, Hk, Hv, D, D, 4, 1e-6,
+            D ** -0.5, address, torch.cuda.current_stream().cuda_stream)
+        torch.cuda.synchronize()
+        assert rc == 0
+        res.append((st, cs, out))
+    assert all(torch.equal(a, b) for a, b in zip(*res))
+    assert (arr == 7).all().item()

@@ -1,6 +1,6 @@
 """GPU parity: the general-shape Gated DeltaNet path (the token-sequential
 kernel the entry points take for shapes outside their tuned kernels: value /
-key head ratios outside {1, 2, 4} or not dividing, dk or dv other than 128,
+key head ratios outside 1-4 (decode) or not dividing, dk or dv other than 128,
 conv kernel widths other than 4). Reference role: the single-workgroup
 fallback of run_linear_delta_decode_gpu (Qwen35HybridTextBackend.cpp:
 1168-1304) and the token loop of run_linear_delta_prefill_gpu_batched.
@@ -60,7 +60,8 @@ def _layer_inputs(seed, B, T, Hk, Hv, dk, dv, K):
 
 LAYER_SHAPES = [
     # (B, Hk, Hv, dk, dv, K)
-    (2, 2, 6, 128, 128, 4),    # Hv / Hk = 3
+    (2, 2, 6, 128, 128, 4),    # Hv / Hk = 3 (the layer decode's tuned kernel)
+    (2, 1, 5, 128, 128, 4),    # Hv / Hk = 5
     (2, 1, 8, 128, 128, 4),    # Hv / Hk = 8
     (1, 3, 4, 128, 128, 4),    # 4 % 3 != 0: the reference's clamp mapping
     (2, 2, 4, 64, 96, 3),      # other head dims and conv width
@@ -91,7 +92,7 @@ def test_generic_layer_decode_steps(B, Hk, Hv, dk, dv, K):
     assert np.array_equal(_np(cs), want_cs), "conv ring must hold the raw inputs bit-exact"
 
 
-@pytest.mark.parametrize("B,Hk,Hv,dk,dv,K", LAYER_SHAPES[:4])
+@pytest.mark.parametrize("B,Hk,Hv,dk,dv,K", LAYER_SHAPES[:5])
 def test_generic_layer_prefill_then_decode(B, Hk, Hv, dk, dv, K):
     """Prefill over T tokens (ragged, and shorter than the ring for one case),
     then decode steps continuing the ring and the state."""
