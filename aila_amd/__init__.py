@@ -96,9 +96,12 @@ def _check(rc: int, what: str) -> None:
 # (whole-layer decode step, back to back calls: 15.4 -> 11.0 us a call).
 def _stream(stream=None):
     import torch
-    if stream is not None:
-        return stream.cuda_stream
-    return torch._C._cuda_getCurrentRawStream(torch.cuda.current_device())
+    if stream is None:
+        raw = getattr(torch._C, "_cuda_getCurrentRawStream", None)   # not public: torch may drop it
+        if raw is not None:
+            return raw(torch.cuda.current_device())
+        stream = torch.cuda.current_stream()
+    return stream.cuda_stream
 
 
 def _ptr(t):

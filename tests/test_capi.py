@@ -53,3 +53,18 @@ def test_argument_validation_runs_before_any_device_work():
     rc = l.aila_hip_deltanet_decode(p, p, p, p, p, None, None, p, p, 1, 3, 4, 320, 128,
                                     1e-6, 0.1, None)
     assert rc == -2 and b"dk=320" in l.aila_hip_last_error()
+
+
+def test_stream_handle(monkeypatch):
+    """A stream's own handle if one is given, else the current one, with and
+    without torch's private accessor of it."""
+    import types
+
+    import torch
+    monkeypatch.setattr(torch.cuda, "current_device", lambda: 0)
+    monkeypatch.setattr(torch.cuda, "current_stream", lambda: types.SimpleNamespace(cuda_stream=21))
+    assert aila_amd._stream(types.SimpleNamespace(cuda_stream=7)) == 7
+    monkeypatch.setattr(torch._C, "_cuda_getCurrentRawStream", lambda device: 20 + device, raising=False)
+    assert aila_amd._stream() == 20
+    monkeypatch.delattr(torch._C, "_cuda_getCurrentRawStream")
+    assert aila_amd._stream() == 21
