@@ -25,7 +25,7 @@
 namespace aila {
 
 // Chunked prefill of the recurrence (deltanet_prefill.hip).
-size_t deltanet_chunk_records_bytes(int B, int T, int Hv, bool split);
+size_t deltanet_chunk_records_bytes(int B, int T, int Hk, int Hv, bool split);
 // conv == nullptr: q, k, v planes; else the layer (q, k, v formed from conv->qkv).
 void launch_deltanet_chunked(const bf16* q, const bf16* k, const bf16* v, const ConvIn* conv, const bf16* a,
                              const bf16* b, int ab_stride, const bf16* dt_bias, const float* A_log, float* state,
@@ -435,7 +435,7 @@ __global__ __launch_bounds__(256) void deltanet_gate_kernel(bf16* __restrict__ o
 
 // The prefill workspace holds the chunk records only (the prep forms q, k,
 // v from the fused rows itself).
-size_t layer_ws_bytes(int B, int T, int Hv) { return deltanet_chunk_records_bytes(B, T, Hv, true); }
+size_t layer_ws_bytes(int B, int T, int Hk, int Hv) { return deltanet_chunk_records_bytes(B, T, Hk, Hv, true); }
 
 }  // namespace
 
@@ -444,7 +444,7 @@ size_t layer_ws_bytes(int B, int T, int Hv) { return deltanet_chunk_records_byte
 extern "C" size_t aila_hip_deltanet_layer_prefill_workspace_size(int B, int T, int Hk, int Hv, int dk, int dv) {
   // 0 also for the shapes that run the sequential general-shape kernel
   if (B <= 0 || T <= 0 || Hk <= 0 || Hv <= 0 || dk != aila::kD || dv != aila::kD || Hv % Hk != 0) return 0;
-  return aila::layer_ws_bytes(B, T, Hv);
+  return aila::layer_ws_bytes(B, T, Hk, Hv);
 }
 
 extern "C" int aila_hip_deltanet_layer_prefill(const void* qkv, int qkv_stride, const void* z, int z_stride,
@@ -493,7 +493,7 @@ extern "C" int aila_hip_deltanet_layer_prefill(const void* qkv, int qkv_stride, 
                    aligned(z, 16) && z_stride % 8 == 0 && aligned(norm_w, 16) && aligned(state, 16) &&
                    aligned(out, 16),
                "deltanet_layer_prefill: misaligned qkv/conv_w/conv_state/z/norm_w/state/out or odd strides");
-  const size_t need = layer_ws_bytes(B, T, Hv);
+  const size_t need = layer_ws_bytes(B, T, Hk, Hv);
   if (!workspace || workspace_bytes < need)
     return set_error(AILA_HIP_EWORKSPACE, "deltanet_layer_prefill: workspace %zu < %zu bytes", workspace_bytes,
                      need);

@@ -1046,14 +1046,11 @@ void launch_scan(const bf16* v, const ConvIn& cv, const unsigned char* records, 
 
 }  // namespace
 
-// Records of the chunked prefill; the sizes callers have allocated since the
-// records also held W and U, which they now only bound.
-size_t deltanet_chunk_records_bytes(int B, int T, int Hv, bool split) {
+// Records of the chunked prefill.
+size_t deltanet_chunk_records_bytes(int B, int T, int Hk, int Hv, bool split) {
   const size_t nch = (static_cast<size_t>(T) + kC - 1) / kC;
-  constexpr size_t kValueHead = 74752, kKeyHead = 32768, kKeyHeadSplit = 49152;
-  static_assert(ChunkRec::kBytes <= kValueHead && KeyRec<false>::kBytes <= kKeyHead && KeyRec<true>::kBytes <= kKeyHeadSplit,
-                "records fit");
-  return static_cast<size_t>(B) * Hv * nch * (kValueHead + (split ? kKeyHeadSplit : kKeyHead));
+  return static_cast<size_t>(B) * nch *
+         (Hv * ChunkRec::kBytes + Hk * (split ? KeyRec<true>::kBytes : KeyRec<false>::kBytes));
 }
 
 // Chunk records + launches of the two kernels; shared by the recurrence
@@ -1077,7 +1074,7 @@ void launch_deltanet_chunked(const bf16* q, const bf16* k, const bf16* v, const 
 extern "C" size_t aila_hip_deltanet_prefill_workspace_size(int B, int T, int Hv, int dk, int dv) {
   // 0 also for the shapes that run the sequential general-shape kernel
   if (B <= 0 || T <= 0 || Hv <= 0 || dk != 128 || dv != 128) return 0;
-  return aila::deltanet_chunk_records_bytes(B, T, Hv, false);
+  return aila::deltanet_chunk_records_bytes(B, T, Hv, Hv, false);   // at most one key head per value head
 }
 
 extern "C" int aila_hip_deltanet_prefill(const void* q, const void* k, const void* v, const void* a,

@@ -351,9 +351,10 @@ int aila_hip_deltanet_layer_decode(const void* qkv, int qkv_stride,
                                    void* stream);
 
 /* Workspace bytes for aila_hip_deltanet_layer_prefill: the per-chunk
- * records (as aila_hip_deltanet_prefill's, plus the key residual; about
- * 121 KiB per sequence, value head and 64-token chunk). 0 for the shapes
- * that run the general-shape kernel (no workspace needed). */
+ * records (as aila_hip_deltanet_prefill's, plus the key residual: 25.25 KiB
+ * per sequence, value head and 64-token chunk and 48 KiB per sequence, key
+ * head and chunk). 0 for the shapes that run the general-shape kernel (no
+ * workspace needed). */
 size_t aila_hip_deltanet_layer_prefill_workspace_size(int B, int T, int Hk,
                                                       int Hv, int dk, int dv);
 
@@ -389,15 +390,16 @@ int aila_hip_deltanet_layer_prefill(const void* qkv, int qkv_stride,
                                     int conv_kernel, float eps, float scale,
                                     void* stream);
 
-/* Workspace bytes for aila_hip_deltanet_prefill (per-chunk W and its
- * residual, U, P, Q, K^T and decay factors, in the scan's operand order;
- * 105 KiB per (sequence, value head, 64-token chunk), of which the key
- * head's K^T and Q parts are used once per key head). 0 for the shapes that
- * run the general-shape kernel. */
+/* Workspace bytes for aila_hip_deltanet_prefill: what the scan reads of each
+ * 64-token chunk, per sequence and value head 25.25 KiB (T = (I + A)^-1 less
+ * its unit diagonal as bf16 hi + residual, P and the row factors) and per
+ * sequence and key head 32 KiB (the K tile and Q), the latter counted for as
+ * many key heads as value heads. 0 for the shapes that run the general-shape
+ * kernel. */
 size_t aila_hip_deltanet_prefill_workspace_size(int B, int T, int Hv, int dk,
                                                 int dv);
 
-/* Chunked Gated DeltaNet prefill (chunk 64, WY/UT form on bf16 MFMA): the
+/* Chunked Gated DeltaNet prefill (chunk 64, UT form on bf16 MFMA): the
  * recurrence of aila_hip_deltanet_decode applied to T tokens, replacing the
  * token-sequential Qwen35HybridTextBackend::run_linear_delta_prefill_gpu_batched
  * (src/models/Qwen35HybridTextBackend.cpp:1306-1508) after conv1d/SiLU.

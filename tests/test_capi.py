@@ -55,6 +55,24 @@ def test_argument_validation_runs_before_any_device_work():
     assert rc == -2 and b"dk=320" in l.aila_hip_last_error()
 
 
+def test_deltanet_workspace_holds_the_records_and_no_more():
+    """25.25 KiB per value head and chunk, 32 (the layer 48) KiB per key head and
+    chunk; one byte less is refused before any device work."""
+    p = ctypes.c_void_p(4096)   # never dereferenced
+    l = aila_amd.lib()
+    for B, T, Hk, Hv in ((1, 1, 1, 1), (1, 4096, 16, 32), (3, 65, 2, 6)):
+        nch = (T + 63) // 64
+        need = aila_amd.deltanet_layer_prefill_workspace_size(B, T, Hk, Hv)
+        assert need == B * nch * (Hv * 25856 + Hk * 49152)
+        ch = 2 * Hk * 128 + Hv * 128
+        assert l.aila_hip_deltanet_layer_prefill(p, ch, p, Hv * 128, p, p, Hv, p, p, 0, None, None, p, p, p, p, need - 1,
+                                                 B, T, Hk, Hv, 128, 128, 4, 1e-6, 0.1, None) == -4
+        need = aila_amd.deltanet_prefill_workspace_size(B, T, Hv, 128, 128)
+        assert need == B * nch * Hv * (25856 + 32768)
+        assert l.aila_hip_deltanet_prefill(p, p, p, p, p, None, None, p, p, p, need - 1, B, T, Hk, Hv, 128, 128, 1e-6,
+                                           0.1, None) == -4
+
+
 def test_stream_handle(monkeypatch):
     """A stream's own handle if one is given, else the current one, with and
     without torch's private accessor of it."""

@@ -92,6 +92,30 @@ def test_prep_either_side_of_its_rule(B, G):
     test_layer_matches_oracle(B, 1, G, 65)
 
 
+@pytest.mark.parametrize("B,Hk,Hv,T", [(1, 1, 1, 1), (2, 2, 4, 129), (1, 1, 8, 300), (3, 11, 33, 65)])
+def test_calls_stay_inside_their_workspace(B, Hk, Hv, T):
+    import torch
+    import aila_amd
+    seed, ch = 44000 + T, 2 * Hk * D + Hv * D
+    q, k = (_t(dg.normal_bf16(seed, i, (B, T, Hk, D))) for i in (0, 1))
+    v, z = (_t(dg.normal_bf16(seed, i, (B, T, Hv, D))) for i in (2, 3))
+    a, b = (_t(dg.normal_bf16(seed, i, (B, T, Hv))) for i in (4, 5))
+    qkv, w = _t(dg.normal_bf16(seed, 6, (B, T, ch))), _t(dg.normal_bf16(seed, 7, (ch, 4), std=0.5))
+    for need, run in (
+            (aila_amd.deltanet_prefill_workspace_size(B, T, Hv, D, D),
+             lambda ws, st: aila_amd.deltanet_prefill(q, k, v, a, b, st, workspace=ws)),
+            (aila_amd.deltanet_layer_prefill_workspace_size(B, T, Hk, Hv),
+             lambda ws, st: aila_amd.deltanet_layer_prefill(qkv, z.view(B, T, Hv * D), a, b, w,
+                                                            torch.zeros((B, 3, ch), device="cuda"), 0,
+                                                            torch.ones(D, device="cuda"), st, Hk, workspace=ws))):
+        print(f"workspace B={B} Hk={Hk} Hv={Hv} T={T} bytes={need}", flush=True)
+        buf = torch.full((need + 65536,), 0xA5, dtype=torch.uint8, device="cuda")
+        st, st2 = (torch.zeros((B, Hv, D, D), device="cuda") for _ in range(2))
+        out = run(buf[:need], st)
+        assert (buf[need:] == 0xA5).all().item()
+        assert torch.equal(out, run(None, st2)) and torch.equal(st, st2)
+
+
 @pytest.mark.parametrize("wide", [False, True])
 @pytest.mark.parametrize("B,Hk", [(1, 1), (3, 2), (8, 16)])
 def test_layer_decode_three_value_heads(B, Hk, wide):
