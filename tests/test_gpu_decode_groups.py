@@ -103,7 +103,10 @@ def test_decode_any_group_device_lengths_and_append(G, Hkv, D):
 
 
 @pytest.mark.parametrize("G,Hkv,D,rot,gate,split", [(5, 8, 128, 128, True, True), (10, 2, 256, 64, False, True),
-                                                     (3, 4, 128, 32, True, False)])
+                                                     (3, 4, 128, 32, True, False)]
+                         # tiles 6 and 7, a tile of 8 with 7 heads (D = 128), and 13 heads as 7 + 6
+                         + [(G, 2, D, D, split, split) for G in (6, 7, 13) for D in (64, 128, 256)
+                            for split in (True, False)])
 def test_fused_prepare_append_any_group(G, Hkv, D, rot, gate, split):
     """QK-norm + RoPE + append + decode in one launch (ElementwiseOps.cpp:
     555-863 then AttentionOps.cpp:499-643) for ratios outside 1, 2, 4, 8."""
