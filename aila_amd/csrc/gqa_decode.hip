@@ -769,18 +769,20 @@ Residency resident_workgroups(int max_per_cu) {
 
 // The plan's workgroups for one round: the same for a contiguous and a paged
 // cache, whose results on the same rows are the same bits only if the rows are
-// split alike. Tiles 1 to 4 at D = 128 take all their occupancy: capped at two a
-// CU a contiguous cache loses more than a paged one gains (120 shapes, 1-32
-// sequences of 1000-32768 rows, all / two a CU: tile 1 geometric mean 5% slower,
+// split alike. Tiles 1 to 4 at D = 128 take all their occupancy (120 shapes, 1-32
+// sequences of 1000-32768 rows, all / two a CU: tile 1 geometric mean 5% faster,
 // B = 22, 1 KV head, 31744 rows 57.9 / 70.0 us; tile 2 5%; tile 3 4%, B = 14, 2 KV
-// heads, 25728 rows 62.4 / 73.4; tile 4 2%, B = 5, 8 KV heads, 6656 rows 27.9 /
-// 32.8; paged, tile 2 6% faster, the others within 2%). Tiles 5 and 6 stream no
+// heads, 25728 rows 62.4 / 73.4; tile 4 2%), tile 2 the paged kernel's three, whose
+// registers do not hold four (600 shapes, three / four a CU: paged 3% faster, the
+// others within 1%). Tiles 5 and 6 stream no
 // faster with three a CU than with two there (tile 6 over two workgroups a KV head
 // 54 / 39 us, paged 40 / 31). At D = 64 tiles 3 and 5 to 7 take three, as tile 8
 // does (paged tile 3 at 16384 rows 13% slower otherwise); 1, 2 and 4 measured up to
 // 10% faster with all theirs.
 Residency resident_for(int D, int tile) {
-  const int cap = D == 64 ? (tile == 3 || tile > 4 ? 3 : 8) : D == 128 && tile > 4 ? 2 : 8;
+  const int cap = D == 64    ? (tile == 3 || tile > 4 ? 3 : 8)
+                  : D == 128 ? (tile > 4 ? 2 : tile == 2 ? 3 : 8)
+                             : 8;
   auto pick = [&](auto d_tag) -> Residency {
     constexpr int DD = decltype(d_tag)::value;
     switch (tile) {
@@ -880,7 +882,13 @@ int gqa_decode_impl(const void* q, const void* k_cache, const void* v_cache, voi
     // 80.7, 2 71.4). More splits take two a CU (B = 4, 11 on 8, window 4462: 8 of 64
     // 45.2, 4 71.9; B = 37, 9 on 2, window 572: 4 of 148 24.2, 2 28.6).
     if (a.win.window > 0 && a.group > 4 && D == 256 && 3 * groups > 2 * resident.cus) resident.per_cu = 1;
-    int want = (resident.per_cu * resident.cus + groups - 1) / groups;
+    const int slots = resident.per_cu * resident.cus, down = slots / groups;
+    int want = (slots + groups - 1) / groups;
+    // Rounding up puts the last few workgroups into a second round; tiles 1 to 4 at D
+    // = 128, planned at all their occupancy, round down where that still fills two
+    // thirds of the slots (B = 28, 3 on 4 KV heads, 6262 rows, paged: 7 splits of 112
+    // workgroups over 768 slots 82.8 us, 6 61.2; 700 shapes: 1-4% faster).
+    if (D == 128 && a.tile <= 4 && want > down && 3 * down * groups >= 2 * slots) want = down;
     want = std::max(1, std::min(want, a.nsplit_max));
     a.split_len = (plan_len + want - 1) / want;
     a.split_len = ((a.split_len + kWaves * kChunk - 1) / (kWaves * kChunk)) * (kWaves * kChunk);

@@ -143,7 +143,7 @@ def test_paged_rejects_bad_arguments():
 
 
 @pytest.mark.parametrize("B,Hkv,D,G,L", [(32, 8, 128, 1, 2100), (32, 8, 128, 2, 4096), (21, 2, 128, 1, 8128), (12, 8, 128, 3, 2304),
-                                         (16, 8, 128, 4, 2000), (10, 8, 128, 7, 2048), (8, 4, 128, 14, 2048),
+                                         (16, 8, 128, 4, 2000), (10, 8, 128, 7, 2048), (8, 4, 128, 14, 2048), (28, 4, 128, 3, 2000), (15, 8, 128, 2, 2000),
                                          (16, 8, 64, 3, 2048), (16, 8, 256, 2, 2048)])
 def test_paged_equals_contiguous_where_the_device_is_full(B, Hkv, D, G, L):
     """Enough sequences and KV heads that the workgroups the device holds, and
