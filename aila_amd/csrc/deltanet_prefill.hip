@@ -31,8 +31,8 @@
 //   is small, forms what the recurrence needs and S does not enter: K, Q,
 //   K K^T and Q K^T once, then To and P for each of its value heads (four waves
 //   per value head).
-// Kernel 2 (deltanet_chunk_scan_kernel): one 8-wave workgroup per (slab of 16
-//   NT columns of dv, value head, sequence) walks the chunks in order with
+// Kernel 2 (deltanet_chunk_scan_kernel): one workgroup of 8 waves (12 at NT = 1)
+//   per (slab of 16 NT columns of dv, value head, sequence) walks the chunks in order with
 //   its state slab in registers of four "state" waves, while four "output"
 //   waves form the outputs beside them, bring the K tiles of later chunks to
 //   LDS by DMA and form the V rows.
@@ -556,7 +556,8 @@ struct OutOps {
   u32x2 v[RAW];      // V input rows (NT = 1: 4 columns, else this lane's NT)
 };
 
-// One workgroup = 8 waves on NT 16-column tiles of one (value head, sequence).
+// One workgroup = 8 waves (12 at NT = 1, with four helpers) on NT 16-column tiles
+// of one (value head, sequence).
 // Waves 0-3 ("state" waves) carry the recurrence: each holds 32 key rows of
 // the slab's state. Waves 4-7 ("output" waves) form the outputs of token tile
 // w4, V of the next chunk, and the DMAs that bring later chunks' K tiles.

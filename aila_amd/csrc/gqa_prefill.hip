@@ -567,8 +567,11 @@ __global__ __launch_bounds__(2 * kThreads, 1) void gqa_prefill_kernel(
 // o *= f when any != 0 (wave-uniform), with the branch inside the statement: as
 // an `if` around all of O the compiler keeps the rescaled O in registers of its
 // own and copies every one of them before the next products (64 v_mov a phase).
-// The rescale, rare, lies out of line. The s_nops cover the distance that matrix
-// instructions need from O's writers and readers.
+// The rescale, rare, lies out of line. The compiler places no waits inside the
+// statement, so the s_nops hold the distances of the longest matrix instructions
+// (16 passes; those of this file take at most 8), whatever the tile shape: 20 wait
+// states from one that wrote O to the products, 8 from the products to one that
+// reads O.
 template <int N>
 __device__ __forceinline__ void rescale_if(uint64_t any, f32x4 (&o)[N], float f) {
   static_assert(N % 2 == 0, "two tiles at a time");
@@ -596,13 +599,15 @@ __device__ __forceinline__ void rescale_if(uint64_t any, f32x4 (&o)[N], float f)
 // key block serves both groups, and the two keep the ping-pong of the kernel
 // above: B runs one phase behind A, a barrier between phases. Against one stream
 // per group this halves the DMAs a workgroup issues (a vector phase of the kernel
-// above spends 550 of its 1260 cycles issuing eight of them at 64 B/clk) and the
+// above spends 465-606 of its some 1000 cycles issuing eight of them) and the
 // K/V bytes it takes from L2, and leaves no partial states to merge; it needs
-// twice the query rows per workgroup.
-// Bound by the operand reads: at 16 query rows a wave every MFMA takes its own
-// KiB from the LDS, 128 KiB in a matrix phase of 1430 cycles with 528 of MFMA (16
-// query heads, S = 8191: 633 -> 587 us, 936 TFLOP/s). D = 128 holds 32 rows a
-// wave and measured no gain (S = 8192: 503 / 511 us).
+// twice the query rows per workgroup. (16 query heads, S = 8191: 633 -> 587 us,
+// 936 TFLOP/s.) D = 128 holds 32 rows a wave and measured no gain (S = 8192: 503 /
+// 511 us).
+// Bound by both phases together: of 1375 cycles a phase the matrix waves take
+// 930-1040 for 528 of MFMA (at 16 query rows a wave every MFMA takes its own KiB
+// from the LDS, 128 KiB a phase), the vector waves beside them 880-990, and the
+// barriers and the wait for the other group the rest.
 //
 // Four buffers each for K and V. In V(j) group A refills K_{j+3} (its buffer
 // held K_{j-1}, which B read last two phases earlier), group B V_{j+2} (buffer
