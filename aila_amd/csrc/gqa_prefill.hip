@@ -76,6 +76,29 @@ __device__ __forceinline__ int swz_v(int r) {
   else return (((r >> 1) & 3) << 1) | ((r >> 3) & 1);
 }
 
+// copy_to_cache of the K/V rows of query blocks qh and ql (bm rows each), to rows
+// from dst0 on: every G-th row from gi, for thread tid0 of nthr.
+template <int D>
+__device__ __forceinline__ void copy_blocks_to_cache(const bf16* Kh, const bf16* Vh, bf16* k_cache, bf16* v_cache,
+                                                     int kv_row_stride, size_t dst0, int ql, int qh, int bm, int S,
+                                                     int gi, int G, int tid0, int nthr) {
+  constexpr int NC = D / 8;
+#pragma unroll 1
+  for (int pass = 0; pass < 2; ++pass) {
+    const int qb = pass == 0 ? qh : ql;
+    if (pass == 1 && ql == qh) break;
+    const int r0 = qb * bm, r1 = min(r0 + bm, S);
+    const int nrow = (r1 - r0 - gi + G - 1) / G;   // rows r0 + gi, r0 + gi + G, ...
+    for (int p = tid0; p < nrow * NC; p += nthr) {
+      const int row = r0 + gi + (p / NC) * G, c = p % NC;
+      const size_t src = static_cast<size_t>(row) * kv_row_stride + c * 8;
+      const size_t dst = (dst0 + row) * D + c * 8;
+      __builtin_nontemporal_store(ld16(Kh + src), reinterpret_cast<u32x4*>(k_cache + dst));
+      __builtin_nontemporal_store(ld16(Vh + src), reinterpret_cast<u32x4*>(v_cache + dst));
+    }
+  }
+}
+
 // One workgroup = two 4-wave groups and one head. It owns a balanced pair of
 // query blocks: light block i and heavy block n-1-i (causal work grows with
 // the block index, so every pair costs n+1 key blocks when start_pos = 0).
@@ -422,26 +445,12 @@ __global__ __launch_bounds__(2 * kThreads, 1) void gqa_prefill_kernel(
     }
   };
 
-  // ---- fused copy_to_cache: this pair's own K/V rows, shared by the G query
-  //      heads of the KV group (head h copies every G-th row from h % G).
+  // ---- fused copy_to_cache: this pair's own K/V rows (head h of a KV group
+  //      copies every G-th row from h % G).
   auto copy_rows_to_cache = [&](int tid0, int nthr) __attribute__((always_inline)) {
-    if (k_cache != nullptr) {
-      const int gi = h % G;
-#pragma unroll 1
-      for (int pass = 0; pass < 2; ++pass) {
-        const int qb = pass == 0 ? qh : ql;
-        if (pass == 1 && ql == qh) break;
-        const int r0 = qb * C::BM, r1 = min(r0 + C::BM, S);
-        const int nrow = (r1 - r0 - gi + G - 1) / G;   // rows r0 + gi, r0 + gi + G, ...
-        for (int p = tid0; p < nrow * C::NC; p += nthr) {
-          const int row = r0 + gi + (p / C::NC) * G, c = p % C::NC;
-          const size_t src = static_cast<size_t>(row) * kv_row_stride + c * 8;
-          const size_t dst = (static_cast<size_t>(kvh) * max_seq + cache_pos + row) * D + c * 8;
-          __builtin_nontemporal_store(ld16(Kh + src), reinterpret_cast<u32x4*>(k_cache + dst));
-          __builtin_nontemporal_store(ld16(Vh + src), reinterpret_cast<u32x4*>(v_cache + dst));
-        }
-      }
-    }
+    if (k_cache != nullptr)
+      copy_blocks_to_cache<D>(Kh, Vh, k_cache, v_cache, kv_row_stride, static_cast<size_t>(kvh) * max_seq + cache_pos, ql,
+                              qh, C::BM, S, h % G, G, tid0, nthr);
   };
 
   // ---- prologue: K_0, V_0, K_1 (+ group A's heavy Q) ------------------------
@@ -904,25 +913,10 @@ __global__ __launch_bounds__(2 * kThreads, 1) void gqa_prefill_shared_kernel(
     store_segment();   // the next segment's first S follows in the same phase
   }
   phase_barrier();
-  // fused copy_to_cache: the K/V rows of this workgroup's query blocks, shared
-  // by the G query heads of the KV group (head h copies every G-th row)
-  if (!KSPLIT && k_cache != nullptr) {
-    const int gi = h % G;
-#pragma unroll 1
-    for (int pass = 0; pass < 2; ++pass) {
-      const int qb = pass == 0 ? qh : ql;
-      if (pass == 1 && ql == qh) break;
-      const int r0 = qb * BMW, r1 = min(r0 + BMW, S);
-      const int nrow = (r1 - r0 - gi + G - 1) / G;   // rows r0 + gi, r0 + gi + G, ...
-      for (int p = threadIdx.x; p < nrow * C::NC; p += 2 * kThreads) {
-        const int row = r0 + gi + (p / C::NC) * G, c = p % C::NC;
-        const size_t src = static_cast<size_t>(row) * kv_row_stride + c * 8;
-        const size_t dst = (static_cast<size_t>(kvh) * max_seq + cache_pos + row) * D + c * 8;
-        __builtin_nontemporal_store(ld16(Kh + src), reinterpret_cast<u32x4*>(k_cache + dst));
-        __builtin_nontemporal_store(ld16(Vh + src), reinterpret_cast<u32x4*>(v_cache + dst));
-      }
-    }
-  }
+  // fused copy_to_cache: the K/V rows of this workgroup's query blocks
+  if (!KSPLIT && k_cache != nullptr)
+    copy_blocks_to_cache<D>(Kh, Vh, k_cache, v_cache, kv_row_stride, static_cast<size_t>(kvh) * max_seq + cache_pos, ql,
+                            qh, BMW, S, h % G, G, threadIdx.x, 2 * kThreads);
   if (grp == 0) phase_barrier();   // group B's last phase
 }
 
